@@ -275,6 +275,25 @@ bool fits_f32(const double* v, int64_t n) {
   }
   return true;
 }
+// Float64 training images that are not FP32-exact: the MFMA scan takes their
+// FP32 rounding (scan_gerr's `rounded` term covers it) when the values keep
+// the range above and no large common offset swamps the differences between
+// windows: the scan's interval is about 2^-14 sqrt(A2 B2) ~ 2^-14 V E[t^2]
+// wide on either side, the distances are of the order of V Var[t], so at
+// E[t^2] <= 32 Var[t] the interval stays near 2^-9 of them and the superset
+// near the band.  Beyond that (and for a constant image) the exhaustive FP64
+// map stays: its time does not depend on the values.
+bool scan_takes_rounded(const double* v, int64_t n) {
+  double s1 = 0.0, s2 = 0.0;
+  for (int64_t i = 0; i < n; i++) {
+    const double x = v[i];
+    if (!(std::fabs(x) <= 0x1p50) || (x != 0.0 && std::fabs(x) < 0x1p-100)) return false;
+    s1 += x;
+    s2 += x * x;
+  }
+  const double m = s1 / (double)n, q = s2 / (double)n;
+  return q <= 32.0 * (q - m * m);
+}
 bool fits_range(const float* v, int64_t n) {
   for (int64_t i = 0; i < n; i++)
     if (!(std::fabs(v[i]) <= 0x1p50f) || (v[i] != 0.0f && std::fabs(v[i]) < 0x1p-100f)) return false;
@@ -296,10 +315,14 @@ bool fits_range(const float* v, int64_t n) {
 //    at most (2^-16 + 2^-17 (1 + 2^-17) + 2^-17) |a||b|
 //    = 2^-15 (1 + 2^-19) |a||b|.  Values are zero or at least 2^-100 in
 //    magnitude (fits_f32 / fits_range), so no part is subnormal.
-double scan_gerr(int64_t nstep, bool split) {
+//  * Rounded (Float64 data taken as t32 = t (1 + d), |d| <= 2^-24, a normal
+//    number): sum |a32||b32| <= (1 + 2^-24)^2 sum |a||b|, and replacing a b by
+//    a32 b32 errs by at most (2^-23 + 2^-48) |a||b|.
+double scan_gerr(int64_t nstep, bool split, bool rounded = false) {
   const double kterms = 16.0 * (double)nstep * (split ? 3.0 : 1.0);
   const double ga = 2.0 * kterms * 0x1p-24 / (1.0 - 2.0 * kterms * 0x1p-24);
-  return 1.02 * ga + (split ? 0x1p-15 * (1.0 + 0x1p-19) : 0.0);
+  const double e = 1.02 * ga + (split ? 0x1p-15 * (1.0 + 0x1p-19) : 0.0);
+  return rounded ? e * (1.0 + 0x1p-22) + 0x1p-22 : e;
 }
 
 void geo_init(IqGeo& g, const int64_t ti[3], const int64_t tile[3]) {
@@ -338,6 +361,7 @@ struct iq_plan {
   double tol = 0.1;
   int naux = 0;
   bool fast = false;
+  bool rounded = false;  // fast, on the FP32 rounding of Float64 data (MFMA scan only)
   bool hard = false;
   bool any_multi = false;
   std::vector<IqStep> steps;
@@ -762,6 +786,7 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
   } else {
     H.ti = pl->mem.upload(tid, tivox, s);
     pl->fast = fits_f32(tid, tivox);
+    if (!pl->fast) pl->fast = pl->rounded = scan_takes_rounded(tid, tivox);
     if (pl->fast) {
       std::vector<float> t32((size_t)tivox);
       for (int64_t i = 0; i < tivox; i++) t32[i] = (float)tid[i];
@@ -897,7 +922,7 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
         pl->mfma = true;
         pl->mfma_lds = lmax;
         pl->mfma_split = !bf16_exact(H.ti32, tivox);
-        pl->mfma_gerr = scan_gerr(H.ktab.nstep, pl->mfma_split);
+        pl->mfma_gerr = scan_gerr(H.ktab.nstep, pl->mfma_split, pl->rounded);
         H.chunks = pl->mem.upload(chunks.data(), chunks.size(), s);
         for (int nw : {2, 3, 4}) {
           if (!pl->lds_nw[nw]) continue;
@@ -923,6 +948,12 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
         }
       }
     }
+  }
+
+  // the VALU scan's bound takes FP32-exact values only
+  if (pl->rounded && !pl->mfma) {
+    pl->fast = false;
+    H.ti32 = nullptr;
   }
 
   // ---- hard and soft data: grids per simulation grid, soft training images shared
@@ -1686,7 +1717,7 @@ void plan_learn(iq_plan* pl, int64_t nsamp, int iters, uint64_t seed) {
   if (nm == 0) bad(IQ_ERR_ARG, "learned proposal: the plan has no overlap mask");
   if (nsamp < IQ_EMB || iters < 0) bad(IQ_ERR_ARG, "learned proposal: need at least 64 samples");
   if (pl->enabled_host.empty()) bad(IQ_ERR_NOCAND, "every candidate pattern is disabled");
-  if (!pl->fast) bad(IQ_ERR_UNSUPPORTED, "learned proposal: training image values must be exact in FP32");
+  if (!pl->fast || pl->rounded) bad(IQ_ERR_UNSUPPORTED, "learned proposal: training image values must be exact in FP32");
   if (!pl->lrn_ready) {
     const int64_t P32 = (g.P + 31) / 32 * 32;
     std::vector<int64_t> wofs(nm), bofs(nm);
@@ -1781,7 +1812,7 @@ struct ConvBuf {
     d.Z = g.ti[2];
     d.N = (int64_t)d.X * d.Y * d.Z;
     x = pl->hd.ti32;
-    if (!x) bad(IQ_ERR_UNSUPPORTED, "convolutional encoder: training image values must be exact in FP32");
+    if (!x || pl->rounded) bad(IQ_ERR_UNSUPPORTED, "convolutional encoder: training image values must be exact in FP32");
     h1 = mem.alloc<float>((size_t)CV_C * d.N);
     h2 = mem.alloc<float>((size_t)CV_C * d.N);
     g1 = mem.alloc<float>((size_t)CV_C * d.N);

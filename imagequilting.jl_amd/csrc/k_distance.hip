@@ -1275,9 +1275,10 @@ k_multi_maps_tiled(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) 
   out[c] = __builtin_fabs((a2 - 2.0 * ab) + b2);
 }
 
-// Plain queries whose training image is not exactly representable in FP32:
-// the overlap map is computed exactly for every candidate, all finite
-// candidates form the superset.
+// Plain queries whose training image the FP32 scans do not take (values out
+// of range, or Float64 values dominated by a common offset): the overlap map
+// is computed exactly for every candidate, all finite candidates form the
+// superset.
 __global__ void __launch_bounds__(256)
 k_band_exact_all(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
   const IqQuery q = qs[blockIdx.y];
