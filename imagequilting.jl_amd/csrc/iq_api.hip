@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "k_distance.hip"
+#include "k_maps.hip"
 #include "k_select.hip"
 #include "k_cut.hip"
 #include "k_learn.hip"
@@ -390,8 +391,14 @@ struct iq_plan {
   int4* dt = nullptr;    // shortlist tiles (all batches of a run)
   int64_t dt_cap = 0;
   size_t cut_lds_max = 0;
-  size_t multi_lds = 0;    // LDS of the tiled multi-source maps (0: gathering kernel)
-  int multi_bx = 16;       // candidate block width of the tiled maps (32 or 16; 16 rows)
+  size_t hard_lds = 0;     // LDS of the tiled hard-data maps (0: gathering kernel)
+  int hard_bx = 16;        // candidate block width of the tiled maps (32 or 16; 16 rows)
+  size_t maps_lds = 0;     // LDS of the exact maps (k_maps_mfma), 0: not used by the plan
+  int maps_steps = 0;      // most steps of any voxel list
+  IqMapTile* dm = nullptr;   // map tiles (all batches of a run)
+  int64_t dm_cap = 0;
+  double* mpack = nullptr;   // their query values in fragment order (one batch at a time)
+  int64_t mpack_cap = 0;
   bool cut_big = false;    // largest slab needs the 512/1024-lane register-resident cut
   int cut_team = 1024;     // its work-items per slab (IQHIP_CUT_TEAM=512: 512)
   int max_nslab = 1;       // most min cuts of any step: the cut launches' grid width
@@ -419,6 +426,8 @@ struct iq_plan {
   hipGraphExec_t gexec[2] = {nullptr, nullptr};
   const IqQuery* gdq[2] = {nullptr, nullptr};
   const int4* gdt[2] = {nullptr, nullptr};
+  const IqMapTile* gdm[2] = {nullptr, nullptr};
+  const double* gmp[2] = {nullptr, nullptr};
   int64_t gnq[2] = {-1, -1};
   int64_t graph_launches = 0;
   // scan profiling
@@ -546,6 +555,91 @@ void tune_scan(iq_plan* pl) {
   if ((int)hq.size() <= 32) pl->nw_tiles[2] = pl->nw_tiles[1];
   HC(hipEventDestroy(a));
   HC(hipEventDestroy(b));
+}
+
+// Voxel lists of the exact maps (k_maps.hip): every mask's, then the whole
+// tile's, cut into chunks whose window region fits MM_LDS (whole planes, as
+// many as fit, else rows of one plane) and steps of 16 voxels inside a chunk.
+void build_map_lists(iq_plan* pl, const std::vector<int32_t>& tvox, int32_t full_off, hipStream_t s) {
+  IqDev& H = pl->hd;
+  const IqGeo& g = pl->geo;
+  const int64_t room = MM_LDS / 8;
+  // voxels of a row, rows and planes of a chunk (rows too long for the room
+  // are cut as well; the region's row pitch is the same for every chunk)
+  const int nx = (int64_t)(MM_BX + g.tile[0] - 1) * MM_BY <= room ? g.tile[0] : (int)(room / MM_BY) - MM_BX + 1;
+  const int RX = MM_BX + nx - 1;
+  const int64_t plane = (int64_t)RX * (MM_BY + g.tile[1] - 1);
+  int ny = 1, nz = 1;
+  if (nx == g.tile[0] && plane <= room) {
+    ny = g.tile[1];
+    nz = (int)std::min<int64_t>(g.tile[2], room / plane);
+  } else if (nx == g.tile[0]) {
+    ny = (int)(room / RX) - MM_BY + 1;
+  }
+  pl->hd.map_rx = RX;
+  std::vector<IqMapChunk> chunks;
+  std::vector<IqMapList> lists;
+  std::vector<int32_t> ofs, vox;
+  const int nm = (int)pl->masks.size();
+  for (int l = 0; l <= nm; l++) {
+    const int off = l < nm ? pl->masks[l].off : full_off, V = l < nm ? pl->masks[l].V : g.tilevox;
+    IqMapList L{(int32_t)chunks.size(), 0, (int32_t)(vox.size() / MM_STEP), 0};
+    int j = 0;
+    while (j < V) {
+      auto coord = [&](int i, int& x, int& y, int& z) {
+        const int t = tvox[off + i];
+        x = t % g.tile[0];
+        y = (t / g.tile[0]) % g.tile[1];
+        z = t / (g.tile[0] * g.tile[1]);
+      };
+      int x, y, z;
+      coord(j, x, y, z);
+      IqMapChunk C{};
+      C.z0 = z / nz * nz;
+      C.nz = std::min(nz, g.tile[2] - C.z0);
+      C.y0 = y / ny * ny;
+      C.x0 = x / nx * nx;
+      C.nx = std::min(nx, g.tile[0] - C.x0);
+      C.ny = std::min(ny, g.tile[1] - C.y0);
+      const int RYc = MM_BY + C.ny - 1;
+      C.s0 = L.ns;
+      int e = j;
+      for (; e < V; e++) {
+        int xe, ye, ze;
+        coord(e, xe, ye, ze);
+        if (ze >= C.z0 + C.nz || ye < C.y0 || ye >= C.y0 + C.ny || xe < C.x0 || xe >= C.x0 + C.nx) break;
+      }
+      for (int s0 = j; s0 < e; s0 += MM_STEP) {
+        int32_t o16[MM_STEP];
+        for (int i = 0; i < MM_STEP; i++) {
+          const int v = s0 + i;
+          o16[i] = -1;
+          if (v < e) {
+            coord(v, x, y, z);
+            o16[i] = x - C.x0 + RX * ((y - C.y0) + RYc * (z - C.z0));
+          }
+          vox.push_back(v < e ? v : -1);
+        }
+        for (int k = 0; k < 4; k++)
+          for (int q = 0; q < 4; q++) ofs.push_back(o16[4 * q + k]);
+        L.ns++;
+      }
+      C.s1 = L.ns;
+      pl->maps_lds = std::max(pl->maps_lds, (size_t)RX * RYc * C.nz * 8);
+      chunks.push_back(C);
+      L.nc++;
+      j = e;
+    }
+    pl->maps_steps = std::max(pl->maps_steps, (int)L.ns);
+    lists.push_back(L);
+  }
+  H.mchunks = pl->mem.upload(chunks.data(), chunks.size(), s);
+  H.mlists = pl->mem.upload(lists.data(), lists.size(), s);
+  H.mofs = (const int4*)pl->mem.upload(ofs.data(), ofs.size(), s);
+  H.mvox = pl->mem.upload(vox.data(), vox.size(), s);
+  HC(hipStreamSynchronize(s));  // the host tables end here
+  if (pl->maps_lds > 64 * 1024)
+    HC(hipFuncSetAttribute((const void*)k_maps_mfma, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl->maps_lds));
 }
 
 // Argument checks of a plan description (the @asserts of iqsim.jl:69-89 as
@@ -1071,32 +1165,32 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
   }
   H.nmap = nmap;
   H.nw32 = nw32;
+  if (pl->any_multi || (!pl->fast && !hmasks.empty())) build_map_lists(pl, tvox, full_off, s);
   if (pl->any_multi) {
-    // tiled exact maps when the candidate block's training-image region, the
-    // query values and their region offsets fit in LDS
-    // (voxel lists as offsets into the staged region; read as scalar loads)
-    // (candidate blocks of 32 x 16 where the region fits, else 16 x 16;
+    // hard-data maps: tiled when some tile holds at least HARD_TILED points
+    // and the candidate block's training-image region fits in LDS (voxel lists
+    // as offsets into the staged region, read as scalar loads; candidate
+    // blocks of 32 x 16 where the region fits, else 16 x 16;
     // IQHIP_MAPS_BX=16 forces the narrow blocks)
+    int hmax = 0;
+    for (const IqStep& st : pl->steps) hmax = std::max(hmax, st.hcnt);
     const char* ebx = std::getenv("IQHIP_MAPS_BX");
     for (int bx : {32, 16}) {
       if (bx == 32 && ebx && std::atoi(ebx) == 16) continue;
+      if (hmax < HARD_TILED && !ebx) break;
       const int RX = bx + g.tile[0] - 1, RY = 16 + g.tile[1] - 1;
       const size_t need = (size_t)RX * RY * g.tile[2] * 8;
-      if (need > 150 * 1024) continue;
-      auto region = [&](const std::vector<int32_t>& tv) {
-        std::vector<int32_t> r(tv.size());
-        for (size_t i = 0; i < tv.size(); i++) {
-          const int t = tv[i], x = t % g.tile[0], y = (t / g.tile[0]) % g.tile[1], z = t / (g.tile[0] * g.tile[1]);
-          r[i] = x + RX * (y + RY * z);
-        }
-        return r;
-      };
-      const std::vector<int32_t> rt = region(tvox), rh = region(htvox);
-      H.rtvox = pl->mem.upload(rt.data(), rt.size(), s);
-      H.rhtvox = rh.empty() ? nullptr : pl->mem.upload(rh.data(), rh.size(), s);
-      pl->multi_lds = need;
-      pl->multi_bx = bx;
-      const void* fn = bx == 32 ? (const void*)k_multi_maps_tiled<32, 16> : (const void*)k_multi_maps_tiled<16, 16>;
+      if (need > 150 * 1024 || htvox.empty()) continue;
+      std::vector<int32_t> rh(htvox.size());
+      for (size_t i = 0; i < htvox.size(); i++) {
+        const int t = htvox[i], x = t % g.tile[0], y = (t / g.tile[0]) % g.tile[1], z = t / (g.tile[0] * g.tile[1]);
+        rh[i] = x + RX * (y + RY * z);
+      }
+      H.rhtvox = pl->mem.upload(rh.data(), rh.size(), s);
+      HC(hipStreamSynchronize(s));
+      pl->hard_lds = need;
+      pl->hard_bx = bx;
+      const void* fn = bx == 32 ? (const void*)k_hard_maps_tiled<32, 16> : (const void*)k_hard_maps_tiled<16, 16>;
       if (need > 64 * 1024) HC(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)need));
       break;
     }
@@ -1198,7 +1292,7 @@ enum { SEL_SCAN = 0, SEL_LEARNED = 1, SEL_CHECK = 2 };
 
 template <typename T>
 void run_batch(iq_plan* pl, const IqQuery* hq, const IqQuery* q, int nq, bool has_plain, bool has_multi, int sel,
-               const int4* tiles, const int4* htiles, int ntiles) {
+               const int4* tiles, const int4* htiles, int ntiles, const IqMapTile* mtiles, int nmtiles) {
   const IqGeo& g = pl->geo;
   hipStream_t s = pl->ctx->stream;
   const IqDev* D = pl->dd;
@@ -1213,6 +1307,15 @@ void run_batch(iq_plan* pl, const IqQuery* hq, const IqQuery* q, int nq, bool ha
     hipLaunchKernelGGL((k_query_prep<T>), dim3(nq, nsrc_prep), dim3(256), 0, s, D, q);
   }
   HCL();
+  if (nmtiles > 0) {
+    // exact maps on the matrix cores: the overlap and soft sources of the
+    // multi-source queries, the overlap of plain queries the scans do not take
+    hipLaunchKernelGGL(k_maps_pack, dim3(pl->maps_steps, nmtiles), dim3(256), 0, s, D, q, mtiles, pl->mpack, pl->maps_steps);
+    HCL();
+    hipLaunchKernelGGL(k_maps_mfma, dim3(nblk(g.dist[0], MM_BX) * nblk(g.dist[1], MM_BY) * (unsigned)g.dist[2], nmtiles),
+                       dim3(512), pl->maps_lds, s, D, q, mtiles, (const double*)pl->mpack, pl->maps_steps);
+    HCL();
+  }
   if (has_plain && sel != SEL_SCAN && ntiles > 0) {
     // shortlist: query encodings -> bracket from a sample -> MFMA scan of the
     // bank keeping what falls in the bracket -> the K best
@@ -1319,7 +1422,7 @@ void run_batch(iq_plan* pl, const IqQuery* hq, const IqQuery* q, int nq, bool ha
       launch_recheck(pl, q, nf, s);
       HCL();
     } else {
-      hipLaunchKernelGGL(k_band_exact_all, dim3(nblk(P, 256), nf), dim3(256), 0, s, D, q);
+      hipLaunchKernelGGL(k_band_all, dim3(nblk(P, 256), nf), dim3(256), 0, s, D, q);
       HCL();
     }
     hipLaunchKernelGGL(k_band_finalize, dim3(nf), dim3(FB), 0, s, D, q, pl->fast ? 1 : 0);
@@ -1330,17 +1433,17 @@ void run_batch(iq_plan* pl, const IqQuery* hq, const IqQuery* q, int nq, bool ha
     }
   }
   if (has_multi) {
-    if (pl->multi_lds > 0) {
-      const int bx = pl->multi_bx;
+    if (pl->hard) {
+      const int bx = pl->hard_bx;
       const unsigned nb = nblk(g.dist[0], bx) * nblk(g.dist[1], 16) * (unsigned)g.dist[2];
-      if (bx == 32)
-        hipLaunchKernelGGL((k_multi_maps_tiled<32, 16>), dim3(nb, nq, 2 + pl->naux), dim3(512), pl->multi_lds, s, D, q);
+      if (pl->hard_lds == 0)
+        hipLaunchKernelGGL(k_hard_maps, dim3(nblk(P, 256), nq), dim3(256), 0, s, D, q);
+      else if (bx == 32)
+        hipLaunchKernelGGL((k_hard_maps_tiled<32, 16>), dim3(nb, nq), dim3(512), pl->hard_lds, s, D, q);
       else
-        hipLaunchKernelGGL((k_multi_maps_tiled<16, 16>), dim3(nb, nq, 2 + pl->naux), dim3(256), pl->multi_lds, s, D, q);
-    } else {
-      hipLaunchKernelGGL(k_multi_maps, dim3(nblk(P, 256), nq, 2 + pl->naux), dim3(256), 0, s, D, q);
+        hipLaunchKernelGGL((k_hard_maps_tiled<16, 16>), dim3(nb, nq), dim3(256), pl->hard_lds, s, D, q);
+      HCL();
     }
-    HCL();
     hipLaunchKernelGGL(k_relax_finalize, dim3(nq), dim3(FB), 0, s, D, q);
     HCL();
   }
@@ -1379,18 +1482,58 @@ struct RunBatch {
   bool plain, multi;
   int64_t toff;
   int nt;
+  int64_t moff;  // map tiles [moff, moff + nm)
+  int nm;
 };
 template <typename T>
 void plan_run_launches(iq_plan* pl, const std::vector<IqQuery>& qs, const std::vector<RunBatch>& batches,
                        const std::vector<int4>& tiles, bool learned);
 void plan_run_finish(iq_plan* pl);
 
+// Map tiles of a batch (and its queries' representatives): the soft maps of
+// its distinct steps, then the overlap maps of its multi-source queries by
+// mask, then, for images the scans do not take, those of its plain queries.
+// Hard and soft maps depend on the step alone, not on the realization, so the
+// first query of a step makes them for all.
+void map_tiles(iq_plan* pl, IqQuery* q, RunBatch& bt, std::vector<IqMapTile>& mtiles) {
+  bt.moff = (int64_t)mtiles.size();
+  const int nm = (int)pl->masks.size();
+  std::map<int32_t, int32_t> first;
+  std::vector<int32_t> reps;
+  std::vector<std::vector<int32_t>> multi((size_t)nm + 1), plain((size_t)nm + 1);
+  for (int i = 0; i < bt.n; i++) {
+    const int mk = pl->steps[q[i].step].mask;
+    if (q[i].multi) {
+      const auto it = first.emplace(q[i].step, i);
+      if (it.second) reps.push_back(i);
+      q[i].rep = q[it.first->second].slot;
+      multi[(size_t)mk + 1].push_back(i);
+    } else if (!pl->fast && mk >= 0) {
+      plain[(size_t)mk + 1].push_back(i);
+    }
+  }
+  auto add = [&](int src, int list, const std::vector<int32_t>& v) {
+    for (size_t i = 0; i < v.size(); i += MM_Q) {
+      IqMapTile T{};
+      T.src = src;
+      T.list = list;
+      T.n = (int32_t)std::min<size_t>(MM_Q, v.size() - i);
+      for (int k = 0; k < T.n; k++) T.q[k] = v[i + k];
+      mtiles.push_back(T);
+    }
+  };
+  for (int a = 0; a < pl->naux; a++) add(2 + a, nm, reps);
+  for (int m = nm; m >= 0; m--) add(0, m - 1, multi[m]);
+  for (int m = nm; m >= 1; m--) add(-1, m - 1, plain[m]);
+  bt.nm = (int)((int64_t)mtiles.size() - bt.moff);
+}
+
 // The query table of a run: wave k of every grid, all realizations, in
 // batches of at most nslots queries (each query's slot is its batch
 // position); with the learned proposal, queries of one mask side by side and
 // the shortlist tiles of each batch.
 void plan_tables(iq_plan* pl, const double* uniforms, const int64_t* forced, bool learned, std::vector<IqQuery>& qs,
-                 std::vector<int4>& tiles, std::vector<RunBatch>& batches) {
+                 std::vector<int4>& tiles, std::vector<IqMapTile>& mtiles, std::vector<RunBatch>& batches) {
   // sampled checks: the batches plan_run will check (every lrn_check-th
   // batch with plain queries) put an evenly strided sample of their queries
   // first, so the sample spans the batch's mask shapes and realizations
@@ -1418,7 +1561,7 @@ void plan_tables(iq_plan* pl, const double* uniforms, const int64_t* forced, boo
         return pl->steps[a.step].mask < pl->steps[b.step].mask;
       });
     for (size_t b0 = 0; b0 < wq.size(); b0 += (size_t)pl->nslots) {
-      RunBatch bt{(int64_t)qs.size(), 0, false, false, 0, 0};
+      RunBatch bt{(int64_t)qs.size(), 0, false, false, 0, 0, 0, 0};
       const size_t b1 = std::min(wq.size(), b0 + (size_t)pl->nslots);
       std::vector<size_t> order(b1 - b0);
       for (size_t k = b0; k < b1; k++) order[k - b0] = k;
@@ -1462,9 +1605,26 @@ void plan_tables(iq_plan* pl, const double* uniforms, const int64_t* forced, boo
           }
         }
       }
+      map_tiles(pl, qs.data() + bt.off, bt, mtiles);
       batches.push_back(bt);
     }
   }
+}
+
+// Uploads a run's map tiles; room for the packed query values of its widest batch.
+void upload_map_tiles(iq_plan* pl, const std::vector<IqMapTile>& mtiles, const std::vector<RunBatch>& batches) {
+  if (mtiles.empty()) return;
+  if ((int64_t)mtiles.size() > pl->dm_cap) {
+    pl->dm = pl->mem.alloc<IqMapTile>(mtiles.size());
+    pl->dm_cap = (int64_t)mtiles.size();
+  }
+  int64_t widest = 0;
+  for (const RunBatch& b : batches) widest = std::max<int64_t>(widest, b.nm);
+  if (widest > pl->mpack_cap) {
+    pl->mpack = pl->mem.alloc<double>((size_t)widest * pl->maps_steps * MM_STEP * MM_Q);
+    pl->mpack_cap = widest;
+  }
+  HC(hipMemcpyAsync(pl->dm, mtiles.data(), mtiles.size() * sizeof(IqMapTile), hipMemcpyHostToDevice, pl->ctx->stream));
 }
 
 template <typename T>
@@ -1489,7 +1649,9 @@ void plan_run(iq_plan* pl, const double* uniforms, const int64_t* forced) {
   std::vector<IqQuery> qs;
   std::vector<int4> tiles;
   std::vector<RunBatch> batches;
-  plan_tables(pl, uniforms, forced, pl->lrn_ready && pl->lrn_on, qs, tiles, batches);
+  std::vector<IqMapTile> mtiles;
+  plan_tables(pl, uniforms, forced, pl->lrn_ready && pl->lrn_on, qs, tiles, mtiles, batches);
+  upload_map_tiles(pl, mtiles, batches);
   if ((int64_t)qs.size() > pl->dq_cap) {
     pl->dq = pl->mem.alloc<IqQuery>(qs.size());
     pl->dq_cap = (int64_t)qs.size();
@@ -1507,7 +1669,8 @@ void plan_run(iq_plan* pl, const double* uniforms, const int64_t* forced) {
   const bool graphable = pl->graphs && !pl->prof && !(learned && pl->lrn_check > 0);
   HC(hipEventRecord(pl->e0, s));
   if (graphable && pl->gexec[gk] &&
-      (pl->gdq[gk] != pl->dq || pl->gdt[gk] != pl->dt || pl->gnq[gk] != (int64_t)qs.size())) {
+      (pl->gdq[gk] != pl->dq || pl->gdt[gk] != pl->dt || pl->gdm[gk] != pl->dm || pl->gmp[gk] != pl->mpack ||
+       pl->gnq[gk] != (int64_t)qs.size())) {
     HC(hipGraphExecDestroy(pl->gexec[gk]));
     pl->gexec[gk] = nullptr;
   }
@@ -1538,6 +1701,8 @@ void plan_run(iq_plan* pl, const double* uniforms, const int64_t* forced) {
       pl->gexec[gk] = ex;
       pl->gdq[gk] = pl->dq;
       pl->gdt[gk] = pl->dt;
+      pl->gdm[gk] = pl->dm;
+      pl->gmp[gk] = pl->mpack;
       pl->gnq[gk] = (int64_t)qs.size();
       HC(hipGraphLaunch(ex, s));
       pl->graph_launches++;
@@ -1587,7 +1752,7 @@ void plan_run_launches(iq_plan* pl, const std::vector<IqQuery>& qs, const std::v
     int sel = SEL_SCAN;
     if (learned && b.plain) sel = (pl->lrn_check > 0 && nplain++ % pl->lrn_check == 0) ? SEL_CHECK : SEL_LEARNED;
     run_batch<T>(pl, qs.data() + b.off, pl->dq + b.off, b.n, b.plain, b.multi, sel, pl->dt + b.toff,
-                 tiles.data() + b.toff, b.nt);
+                 tiles.data() + b.toff, b.nt, pl->dm + b.moff, b.nm);
     if (sel == SEL_CHECK) {
       // the full scan decided this batch: stop using the shortlist once its
       // cumulative recall on the exact bands falls below the threshold.  The
@@ -2173,7 +2338,9 @@ void conv_harvest(iq_plan* pl, int64_t nq_total, int topn, int nhard, int nrand,
   std::vector<IqQuery> qs;
   std::vector<int4> tiles;
   std::vector<RunBatch> batches;
-  plan_tables(pl, U.data(), nullptr, false, qs, tiles, batches);
+  std::vector<IqMapTile> mtiles;
+  plan_tables(pl, U.data(), nullptr, false, qs, tiles, mtiles, batches);
+  upload_map_tiles(pl, mtiles, batches);
   auto eligible = [&](const IqQuery& q) {
     const IqStep& st = pl->steps[q.step];
     return !q.multi && st.active && st.mask >= 0;
@@ -2210,7 +2377,8 @@ void conv_harvest(iq_plan* pl, int64_t nq_total, int topn, int nhard, int nrand,
       left -= take;
       if (!pool.empty()) harvest_queries<T>(pl, pool, topn, nrand, rng, ws, set);
     }
-    run_batch<T>(pl, qs.data() + bt.off, pl->dq + bt.off, bt.n, bt.plain, bt.multi, SEL_SCAN, nullptr, nullptr, 0);
+    run_batch<T>(pl, qs.data() + bt.off, pl->dq + bt.off, bt.n, bt.plain, bt.multi, SEL_SCAN, nullptr, nullptr, 0, pl->dm + bt.moff,
+                 bt.nm);
   }
   HC(hipStreamSynchronize(s));
   int32_t code = 0;

@@ -67,8 +67,31 @@ struct IqQuery {
   int32_t real;    // realization
   int32_t slot;    // scratch slot
   int32_t multi;   // 1: relaxation / tau model over several sources
+  int32_t rep;     // multi: slot of the batch's first query of this step, which holds the step's hard and soft maps
+  int32_t pad_;
   double u;        // uniform of the draw
   int64_t forced;  // pick to replay, or -1
+};
+
+// Exact FP64 maps on the matrix cores (k_maps.hip).  A voxel list (a mask's
+// voxels, or the whole tile) in steps of 16 voxels; chunks are ranges of steps
+// whose window region is staged together: tile planes [z0, z0 + nz), rows
+// [y0, y0 + ny), voxels [x0, x0 + nx) of a row.
+struct IqMapChunk {
+  int32_t z0, nz, y0, ny, x0, nx;
+  int32_t s0, s1;  // steps [s0, s1) of the list
+};
+struct IqMapList {
+  int32_t c0, nc;  // its chunks
+  int32_t s0, ns;  // its first entry in the step tables, its steps
+};
+// Up to 16 queries (batch positions) of one voxel list and one image.
+struct IqMapTile {
+  int32_t src;   // 0 overlap, 2 + a soft pair a, -1 overlap of plain queries (into dexact)
+  int32_t list;  // mask, or the number of masks for the whole tile; -1: no overlap (distance 0)
+  int32_t n;
+  int32_t pad_;
+  int32_t q[16];
 };
 
 // MFMA scan: the K dimension is a list of 8-voxel chunks over the union of
@@ -153,8 +176,7 @@ struct IqDev {
   const int32_t* toff;   // matching training-image offsets
   const int32_t* htvox;  // hard voxels per step
   const int32_t* htoff;
-  const int32_t* rtvox;   // tvox entries as offsets into the tiled multi-map's staged region
-  const int32_t* rhtvox;  // htvox entries likewise
+  const int32_t* rhtvox;  // htvox entries as offsets into the tiled hard map's staged region
   int32_t full_off;
   const double* const* a2maps;
   const float* const* a2f;  // FP32 copies of a2maps, NaN where the window is disabled
@@ -189,6 +211,11 @@ struct IqDev {
   // multi-source selection (relaxation.jl / taumodel.jl), per slot
   double* maps;      int32_t nmap;         // nmap maps of P: 0 overlap, 1 hard, 2+a soft
   uint32_t* bits;    int64_t nw32;         // nmap bitmaps of P bits
+  int32_t map_rx;                          // row pitch of the exact maps' staged region
+  const IqMapChunk* mchunks;               // exact maps: voxel lists of the masks, then of the whole tile
+  const IqMapList* mlists;
+  const int4* mofs;                        // per step and voxel mod 4: region offsets of its four voxels (-1: pad)
+  const int32_t* mvox;                     // per step: 16 list positions (-1: pad)
   int32_t* ev;                             // pattern database (P)
   double* vals;                            // P
   // MFMA scan

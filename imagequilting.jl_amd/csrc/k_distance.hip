@@ -113,11 +113,11 @@ __device__ __forceinline__ void query_prep_body(const IqDev* __restrict__ D, con
       D->nsup[slot] = 0;
     }
   } else if (src == 1) {
-    if (!q.multi || !st.hard) return;
+    if (!q.multi || q.rep != q.slot || !st.hard) return;
     V = st.hcnt;
     tv = D->htvox + st.hoff;
   } else {
-    if (!q.multi) return;
+    if (!q.multi || q.rep != q.slot) return;
     V = g.tilevox;
     tv = D->tvox + D->full_off;
   }
@@ -1121,109 +1121,74 @@ k_band_recheck_lanes(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs
 }
 
 // ---------------------------------------------------------------------------
-// Exact maps for the multi-source selection (relaxation): one work-item per
-// candidate, grid (candidate blocks, query, source).  Source 0 uses the A2 map
-// of its mask (or is identically 0 without a mask), the hard source chains
-// A2, soft sources use the full-tile A2 map of their auxiliary image.
-// Disabled candidates are +inf (iqsim.jl:207,217,226).
+// Exact maps of the hard-data source (relaxation): one work-item per
+// candidate, grid (candidate blocks, query).  Every tile has its own list of
+// hard voxels, and A2 is chained along with AB.  The map depends on the step
+// alone, so the batch's first query of a step makes it for all realizations.
+// Disabled candidates are +inf (iqsim.jl:207,217,226).  This form gathers the
+// windows from the image: a tile usually holds a handful of points, for which
+// staging its windows' region (k_hard_maps_tiled) costs more than it saves.
 // ---------------------------------------------------------------------------
+#define HARD_TILED 48  // hard points of a tile from which the plan uses the tiled form
 __global__ void __launch_bounds__(256)
-k_multi_maps(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
+k_hard_maps(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
   const IqQuery q = qs[blockIdx.y];
-  if (!q.multi) return;
-  const int src = blockIdx.z;
   const IqStep& st = D->steps[q.step];
-  if (src == 1 && !st.hard) return;
+  if (!q.multi || q.rep != q.slot || !st.hard) return;
   const IqGeo& g = D->g;
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= g.P) return;
   const int64_t slot = q.slot;
-  double* out = D->maps + (slot * D->nmap + src) * g.P;
+  double* out = D->maps + (slot * D->nmap + 1) * g.P;
   if (D->disabled[c]) { out[c] = __builtin_inf(); return; }
-  int V;
-  const int32_t* toff;
-  const double* a2map = nullptr;
-  const double* img64 = nullptr;
-  if (src == 0) {
-    if (st.mask < 0) { out[c] = 0.0; return; }
-    const IqMask& m = D->masks[st.mask];
-    V = m.V; toff = D->toff + m.off; a2map = D->a2maps[m.a2];
-  } else if (src == 1) {
-    V = st.hcnt; toff = D->htoff + st.hoff;
-  } else {
-    V = g.tilevox; toff = D->toff + D->full_off; a2map = D->a2soft[src - 2]; img64 = D->auxti[src - 2];
-  }
-  const double* kv = D->kv + slot * D->kv_stride + (int64_t)src * g.tilevox;
-  const double b2 = D->b2[slot * (2 + D->naux) + src];
+  const int V = st.hcnt;
+  const int32_t* toff = D->htoff + st.hoff;
+  const double* kv = D->kv + slot * D->kv_stride + (int64_t)g.tilevox;
+  const double b2 = D->b2[slot * (2 + D->naux) + 1];
   int cx = (int)(c % g.dist[0]), cy = (int)((c / g.dist[0]) % g.dist[1]);
   int cz = (int)(c / ((int64_t)g.dist[0] * g.dist[1]));
   const int64_t base = iq_lin3(g.ti, cx, cy, cz);
   double a2 = 0.0, ab = 0.0;
-  if (img64) {
-    for (int j = 0; j < V; j++) ab = __builtin_fma(img64[base + toff[j]], kv[j], ab);
-  } else if (D->ti_f32) {
+  if (D->ti_f32) {
     const float* ti = (const float*)D->ti;
     for (int j = 0; j < V; j++) {
       double t = (double)ti[base + toff[j]];
-      if (!a2map) a2 = __builtin_fma(t, t, a2);
+      a2 = __builtin_fma(t, t, a2);
       ab = __builtin_fma(t, kv[j], ab);
     }
   } else {
     const double* ti = (const double*)D->ti;
     for (int j = 0; j < V; j++) {
       double t = ti[base + toff[j]];
-      if (!a2map) a2 = __builtin_fma(t, t, a2);
+      a2 = __builtin_fma(t, t, a2);
       ab = __builtin_fma(t, kv[j], ab);
     }
   }
-  if (a2map) a2 = a2map[c];
   out[c] = __builtin_fabs((a2 - 2.0 * ab) + b2);
 }
 
-// Tiled form of k_multi_maps: a workgroup of MX x MY work-items owns MX x MY
-// candidates at one z (32 x 16 where the region fits, else 16 x 16: rows of
-// 32 consecutive candidates keep a half-wavefront's 8-byte reads on distinct
-// LDS banks, and 512-wide groups hold more wavefronts per compute unit); the training-image (or auxiliary-TI) region their windows cover is
-// staged in LDS as FP64, so every work-item's chain (same ascending order,
-// same operations as k_multi_maps) reads LDS instead of gathering from HBM.
-// The query values and the voxels' region offsets (prepared per plan) are
-// the same for every work-item and come through scalar loads.  Grid: (x
-// blocks * y blocks * dist z, query, source); LDS = the region (the host
+// Tiled form for tiles with many hard points: a workgroup of MX x MY
+// work-items owns MX x MY candidates at one z (32 x 16 where the region fits,
+// else 16 x 16: rows of 32 consecutive candidates keep a half-wavefront's
+// 8-byte reads on distinct LDS banks, and 512-wide groups hold more wavefronts
+// per compute unit); the training-image region their windows cover is staged
+// in LDS as FP64.  The query values and the voxels' region offsets (prepared
+// per plan) are the same for every work-item and come through scalar loads.
+// Grid: (x blocks * y blocks * dist z, query); LDS = the region (the host
 // checks it fits).
 template <int MT_X, int MT_Y>
 __global__ void __launch_bounds__(MT_X * MT_Y)
-k_multi_maps_tiled(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
+k_hard_maps_tiled(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
   extern __shared__ double mreg[];
   const IqQuery q = qs[blockIdx.y];
-  if (!q.multi) return;
-  const int src = blockIdx.z;
   const IqStep& st = D->steps[q.step];
-  if (src == 1 && !st.hard) return;
+  if (!q.multi || q.rep != q.slot || !st.hard) return;
   const IqGeo& g = D->g;
   const int nbx = (g.dist[0] + MT_X - 1) / MT_X, nby = (g.dist[1] + MT_Y - 1) / MT_Y;
   const int bx = blockIdx.x % nbx, by = (blockIdx.x / nbx) % nby, cz = blockIdx.x / (nbx * nby);
   const int64_t slot = q.slot;
-  double* out = D->maps + (slot * D->nmap + src) * g.P;
-  int V;
-  const int32_t* rtv;
-  const double* a2map = nullptr;
-  const double* img64 = nullptr;
-  if (src == 0) {
-    if (st.mask < 0) {
-      const int cx = bx * MT_X + (threadIdx.x % MT_X), cy = by * MT_Y + (threadIdx.x / MT_X);
-      if (cx < g.dist[0] && cy < g.dist[1]) {
-        const int64_t c = iq_lin3(g.dist, cx, cy, cz);
-        out[c] = D->disabled[c] ? __builtin_inf() : 0.0;
-      }
-      return;
-    }
-    const IqMask& m = D->masks[st.mask];
-    V = m.V; rtv = D->rtvox + m.off; a2map = D->a2maps[m.a2];
-  } else if (src == 1) {
-    V = st.hcnt; rtv = D->rhtvox + st.hoff;
-  } else {
-    V = g.tilevox; rtv = D->rtvox + D->full_off; a2map = D->a2soft[src - 2]; img64 = D->auxti[src - 2];
-  }
+  double* out = D->maps + (slot * D->nmap + 1) * g.P;
+  const int V = st.hcnt;
   const int RX = MT_X + g.tile[0] - 1, RY = MT_Y + g.tile[1] - 1, RZ = g.tile[2];
   const int nreg = RX * RY * RZ;
   double* reg = mreg;
@@ -1234,81 +1199,31 @@ k_multi_maps_tiled(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) 
     double v = 0.0;
     if (gx < g.ti[0] && gy < g.ti[1]) {
       const int64_t o = iq_lin3(g.ti, gx, gy, gz);
-      v = img64 ? img64[o] : (D->ti_f32 ? (double)((const float*)D->ti)[o] : ((const double*)D->ti)[o]);
+      v = D->ti_f32 ? (double)((const float*)D->ti)[o] : ((const double*)D->ti)[o];
     }
     reg[i] = v;
   }
   // query values and region offsets are the same for every work-item:
   // constant-address loads (scalar unit, no LDS traffic)
-  const auto kq = iq_const(D->kv + slot * D->kv_stride + (int64_t)src * g.tilevox);
-  const auto ro = iq_const(rtv);
+  const auto kq = iq_const(D->kv + slot * D->kv_stride + (int64_t)g.tilevox);
+  const auto ro = iq_const(D->rhtvox + st.hoff);
   __syncthreads();
   const int lx = threadIdx.x % MT_X, ly = threadIdx.x / MT_X;
   const int cx = gx0 + lx, cy = gy0 + ly;
   if (cx >= g.dist[0] || cy >= g.dist[1]) return;
   const int64_t c = iq_lin3(g.dist, cx, cy, cz);
   if (D->disabled[c]) { out[c] = __builtin_inf(); return; }
-  const double b2 = D->b2[slot * (2 + D->naux) + src];
+  const double b2 = D->b2[slot * (2 + D->naux) + 1];
   const double* r0 = reg + lx + RX * ly;
   double a2 = 0.0, ab = 0.0;
   int j = 0;
-  if (!a2map) {
-    for (; j + 8 <= V; j += 8) {
-      double t[8], u[8];
+  for (; j + 8 <= V; j += 8) {
+    double t[8], u[8];
 #pragma unroll
-      for (int i = 0; i < 8; i++) { t[i] = r0[ro[j + i]]; u[i] = kq[j + i]; }
+    for (int i = 0; i < 8; i++) { t[i] = r0[ro[j + i]]; u[i] = kq[j + i]; }
 #pragma unroll
-      for (int i = 0; i < 8; i++) { a2 = __builtin_fma(t[i], t[i], a2); ab = __builtin_fma(t[i], u[i], ab); }
-    }
-    for (; j < V; j++) { const double t = r0[ro[j]]; a2 = __builtin_fma(t, t, a2); ab = __builtin_fma(t, kq[j], ab); }
-  } else {
-    for (; j + 8 <= V; j += 8) {
-      double t[8], u[8];
-#pragma unroll
-      for (int i = 0; i < 8; i++) { t[i] = r0[ro[j + i]]; u[i] = kq[j + i]; }
-#pragma unroll
-      for (int i = 0; i < 8; i++) ab = __builtin_fma(t[i], u[i], ab);
-    }
-    for (; j < V; j++) ab = __builtin_fma(r0[ro[j]], kq[j], ab);
-    a2 = a2map[c];
+    for (int i = 0; i < 8; i++) { a2 = __builtin_fma(t[i], t[i], a2); ab = __builtin_fma(t[i], u[i], ab); }
   }
+  for (; j < V; j++) { const double t = r0[ro[j]]; a2 = __builtin_fma(t, t, a2); ab = __builtin_fma(t, kq[j], ab); }
   out[c] = __builtin_fabs((a2 - 2.0 * ab) + b2);
-}
-
-// Plain queries whose training image the FP32 scans do not take (values out
-// of range, or Float64 values dominated by a common offset): the overlap map
-// is computed exactly for every candidate, all finite candidates form the
-// superset.
-__global__ void __launch_bounds__(256)
-k_band_exact_all(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
-  const IqQuery q = qs[blockIdx.y];
-  const IqStep& st = D->steps[q.step];
-  if (q.multi || st.mask < 0) return;
-  const IqGeo& g = D->g;
-  const int64_t slot = q.slot;
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const IqMask& m = D->masks[st.mask];
-  bool in = false;
-  double d = __builtin_inf();
-  if (c < g.P && !D->disabled[c]) {
-    const int32_t* toff = D->toff + m.off;
-    const double* kv = D->kv + slot * D->kv_stride;
-    int cx = (int)(c % g.dist[0]), cy = (int)((c / g.dist[0]) % g.dist[1]);
-    int cz = (int)(c / ((int64_t)g.dist[0] * g.dist[1]));
-    const int64_t base = iq_lin3(g.ti, cx, cy, cz);
-    const double* ti = (const double*)D->ti;
-    double ab = 0.0;
-    for (int j = 0; j < m.V; j++) ab = __builtin_fma(ti[base + toff[j]], kv[j], ab);
-    d = __builtin_fabs((D->a2maps[m.a2][c] - 2.0 * ab) + D->b2[slot * (2 + D->naux)]);
-    D->dexact[slot * g.P + c] = d;
-    in = true;
-  }
-  const unsigned long long bal = __ballot(in);
-  if ((threadIdx.x & 63) == 0 && (c >> 6) < D->nw64) D->bitmap[slot * D->nw64 + (c >> 6)] = bal;
-  unsigned long long bits = in ? (unsigned long long)__double_as_longlong(d) : 0x7ff0000000000000ull;
-  for (int o = 32; o > 0; o >>= 1) {
-    unsigned long long other = __shfl_xor(bits, o);
-    bits = other < bits ? other : bits;
-  }
-  if ((threadIdx.x & 63) == 0 && bal) atomicMin(&D->gmin64[slot], bits);
 }

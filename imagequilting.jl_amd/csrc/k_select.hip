@@ -867,10 +867,10 @@ k_relax_finalize(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
   int nsrc = 0;
   if (threadIdx.x == 0) {
     int k = 0;
-    if (st.hard) mp[k++] = D->maps + (slot * D->nmap + 1) * g.P;
+    if (st.hard) mp[k++] = D->maps + (q.rep * (int64_t)D->nmap + 1) * g.P;
     mp[k++] = D->maps + (slot * D->nmap + 0) * g.P;
     for (int a = 0; a < D->naux; a++) {
-      mp[k++] = D->maps + (slot * D->nmap + 2 + a) * g.P;
+      mp[k++] = D->maps + (q.rep * (int64_t)D->nmap + 2 + a) * g.P;
     }
     sh.flag = k;
   }
