@@ -57,13 +57,41 @@ struct iq_ctx {
 };
 
 namespace {
-// LDS bytes of one slab's cut of n interior nodes: register-resident form
-// (at most 4 CB nodes, or any slab of a plan run by the large-slab kernel),
-// LDS-resident form (up to IQ_PR_NLDS), else none (global scratch)
-size_t cut_lds_bytes(int64_t n, bool big) {
-  if (n <= 4 * CB || (big && n <= CUT_BIG_MAX)) return (size_t)n * CUT_FAST_NODE_BYTES;
-  if (n <= IQ_PR_NLDS) return (size_t)n * CUT_NODE_BYTES;
-  return 0;
+// Work-items of a cut launch whose largest slab has n interior nodes: a lane
+// per node up to `most` (CUT_TEAM_MAX, or 512 under IQHIP_CUT_TEAM), then two
+// or three nodes a lane (1,536 nodes on 1,024 lanes, half of them with two: 489
+// us per 96 slabs, against 548 us on 768 lanes with two each) ...
+int cut_team(int64_t n, int most = CUT_TEAM_MAX) {
+  if (n > CUT_REG_MAX) return 256;
+  return (int)std::min<int64_t>(most, std::max<int64_t>(64, (n + 63) / 64 * 64));
+}
+
+// ... and its nodes a lane (0: node state in global scratch)
+int cut_npt(int64_t n, int team) { return n > CUT_REG_MAX ? 0 : (int)std::max<int64_t>(1, (n + team - 1) / team); }
+
+template <typename T>
+auto cut_kernel(int npt) {
+  switch (npt) {
+    case 0: return k_graphcut<T, 0>;
+    case 1: return k_graphcut<T, 1>;
+    case 2: return k_graphcut<T, 2>;
+    default: return k_graphcut<T, 3>;
+  }
+}
+template <typename T>
+auto cut_host_kernel(int npt) {
+  switch (npt) {
+    case 0: return k_graphcut_host<T, 0>;
+    case 1: return k_graphcut_host<T, 1>;
+    case 2: return k_graphcut_host<T, 2>;
+    default: return k_graphcut_host<T, 3>;
+  }
+}
+
+// LDS bytes of one slab's cut of n interior nodes (register-resident form;
+// larger slabs keep their state in global scratch)
+size_t cut_lds_bytes(int64_t n) {
+  return n <= CUT_REG_MAX ? (size_t)((n + 63) / 64 * 64) * CUT_FAST_NODE_BYTES : 0;
 }
 
 int fail(const iq_ctx* ctx, int code, const std::string& msg) {
@@ -399,8 +427,8 @@ struct iq_plan {
   int64_t dm_cap = 0;
   double* mpack = nullptr;   // their query values in fragment order (one batch at a time)
   int64_t mpack_cap = 0;
-  bool cut_big = false;    // largest slab needs the 512/1024-lane register-resident cut
-  int cut_team = 1024;     // its work-items per slab (IQHIP_CUT_TEAM=512: 512)
+  int cut_npt = 1;         // interior nodes a lane of a cut (0: global scratch)
+  int cut_team = 256;      // work-items of a cut (IQHIP_CUT_TEAM=512: at most 512)
   int max_nslab = 1;       // most min cuts of any step: the cut launches' grid width
   bool cut_wave = false;   // every slab fits the one-wavefront cut
   std::vector<int32_t> enabled_host;
@@ -1108,16 +1136,13 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
       const IqSlab& sl = st.slab[q];
       maxn = std::max(maxn, (int64_t)sl.sz[0] * sl.sz[1] * sl.sz[2] / sl.sz[sl.dim] * std::max(0, sl.sz[sl.dim] - 2));
     }
-  pl->cut_big = maxn > 4 * CB && maxn <= CUT_BIG_MAX;
   for (const IqStep& st : pl->steps) pl->max_nslab = std::max(pl->max_nslab, st.ncut);
-  for (const IqStep& st : pl->steps)
-    for (int q = 0; q < st.nslab; q++) {
-      const IqSlab& sl = st.slab[q];
-      const int64_t n = (int64_t)sl.sz[0] * sl.sz[1] * sl.sz[2] / sl.sz[sl.dim] * std::max(0, sl.sz[sl.dim] - 2);
-      pl->cut_lds_max = std::max(pl->cut_lds_max, cut_lds_bytes(n, pl->cut_big));
-    }
+  pl->cut_lds_max = cut_lds_bytes(maxn);
   pl->cut_wave = maxn <= CUT_WAVE_MAX;
-  const int64_t cutper = (maxn > IQ_PR_NLDS && !pl->cut_big) ? maxn * CUT_NODE_BYTES : 0;
+  const char* et = std::getenv("IQHIP_CUT_TEAM");
+  pl->cut_team = cut_team(maxn, et && std::atoi(et) == 512 && maxn <= 3 * 512 ? 512 : CUT_TEAM_MAX);
+  pl->cut_npt = cut_npt(maxn, pl->cut_team);
+  const int64_t cutper = maxn > CUT_REG_MAX ? maxn * CUT_NODE_BYTES : 0;
   size_t per_slot = (size_t)nmap * g.tilevox * 8 + (size_t)kmax * 4 + 64 + (size_t)P * (4 + 8 + 4 + 4 + 16) + nw64 * 8 +
                     (size_t)IQ_SORT_MAX * 12 + (size_t)(nw64 + 1) * 8 + (size_t)IQ_MAX_SLAB * g.tilevox +
                     (size_t)IQ_MAX_SLAB * cutper;
@@ -1211,7 +1236,6 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
   H.rc_small = RC_SMALL;
   if (const char* erc = std::getenv("IQHIP_RC_SMALL")) H.rc_small = std::max(0, std::atoi(erc));
   if (const char* eg = std::getenv("IQHIP_GRAPH")) pl->graphs = std::atoi(eg) != 0;
-  if (const char* et = std::getenv("IQHIP_CUT_TEAM")) pl->cut_team = std::atoi(et) == 512 ? 512 : 1024;
   // the exact recheck runs a lane per superset member (k_band_recheck_lanes;
   // measured faster than a wavefront per member at 720- and 4,736-voxel
   // masks); IQHIP_RECHECK=groups selects the wavefront-per-member kernel
@@ -1231,12 +1255,8 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
   HC(hipEventCreate(&pl->e0));
   HC(hipEventCreate(&pl->e1));
   if (pl->cut_lds_max > 64 * 1024) {
-    HC(hipFuncSetAttribute((const void*)k_graphcut<float>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl->cut_lds_max));
-    HC(hipFuncSetAttribute((const void*)k_graphcut<double>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl->cut_lds_max));
-    HC(hipFuncSetAttribute((const void*)k_graphcut_big<float, 512>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl->cut_lds_max));
-    HC(hipFuncSetAttribute((const void*)k_graphcut_big<double, 512>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl->cut_lds_max));
-    HC(hipFuncSetAttribute((const void*)k_graphcut_big<float, 1024>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl->cut_lds_max));
-    HC(hipFuncSetAttribute((const void*)k_graphcut_big<double, 1024>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl->cut_lds_max));
+    const void* fn = pl->dtype == IQ_F32 ? (const void*)cut_kernel<float>(pl->cut_npt) : (const void*)cut_kernel<double>(pl->cut_npt);
+    HC(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl->cut_lds_max));
   }
   if (pl->dtype == IQ_F32) tune_scan<float>(pl);
   else tune_scan<double>(pl);
@@ -1459,12 +1479,8 @@ void run_batch(iq_plan* pl, const IqQuery* hq, const IqQuery* q, int nq, bool ha
   }
   if (pl->cut_wave)
     hipLaunchKernelGGL((k_graphcut_wave<T>), dim3(pl->max_nslab, nq), dim3(64), pl->cut_lds_max, s, D, q);
-  else if (pl->cut_big && pl->cut_team == 1024)
-    hipLaunchKernelGGL((k_graphcut_big<T, 1024>), dim3(pl->max_nslab, nq), dim3(1024), pl->cut_lds_max, s, D, q);
-  else if (pl->cut_big)
-    hipLaunchKernelGGL((k_graphcut_big<T, CB_BIG>), dim3(pl->max_nslab, nq), dim3(CB_BIG), pl->cut_lds_max, s, D, q);
   else
-    hipLaunchKernelGGL((k_graphcut<T>), dim3(pl->max_nslab, nq), dim3(CB), pl->cut_lds_max, s, D, q);
+    hipLaunchKernelGGL(cut_kernel<T>(pl->cut_npt), dim3(pl->max_nslab, nq), dim3(pl->cut_team), pl->cut_lds_max, s, D, q);
   HCL();
   if (pl->prof) {
     HC(hipEventRecord(pl->cut_ev[pl->cut_used + 1], s));
@@ -2691,14 +2707,16 @@ int64_t cut_check(int dtype, const int64_t dims[3], int dim) {
 }
 
 // A, B, keep: device slabs of extents dims; gscr: node state for slabs of
-// more than IQ_PR_NLDS interior nodes (n * CUT_NODE_BYTES), else unused;
+// more than CUT_REG_MAX interior nodes (n * CUT_NODE_BYTES), else unused;
 // err: device status word, zero before the launch.
 void cut_launch(hipStream_t s, const void* dA, const void* dB, int dtype, const int64_t dims[3], int dim, int64_t n,
                 uint8_t* keep, char* gscr, int32_t* err) {
-  const size_t lds = cut_lds_bytes(n, false);
+  const size_t lds = cut_lds_bytes(n);
+  const int team = cut_team(n);
+  const int npt = cut_npt(n, team);
   if (lds > 64 * 1024) {
-    HC(hipFuncSetAttribute((const void*)k_graphcut_host<float>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    HC(hipFuncSetAttribute((const void*)k_graphcut_host<double>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    const void* fn = dtype == IQ_F32 ? (const void*)cut_host_kernel<float>(npt) : (const void*)cut_host_kernel<double>(npt);
+    HC(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   }
   const int s0 = (int)dims[0], s1 = (int)dims[1], s2 = (int)dims[2];
   if (n <= CUT_WAVE_MAX && dtype == IQ_F32)
@@ -2708,10 +2726,10 @@ void cut_launch(hipStream_t s, const void* dA, const void* dB, int dtype, const 
     hipLaunchKernelGGL((k_graphcut_host_wave<double>), dim3(1), dim3(64), lds, s, (const double*)dA,
                        (const double*)dB, s0, s1, s2, dim, keep, err);
   else if (dtype == IQ_F32)
-    hipLaunchKernelGGL((k_graphcut_host<float>), dim3(1), dim3(CB), lds, s, (const float*)dA, (const float*)dB,
+    hipLaunchKernelGGL(cut_host_kernel<float>(npt), dim3(1), dim3(team), lds, s, (const float*)dA, (const float*)dB,
                        s0, s1, s2, dim, keep, gscr, err);
   else
-    hipLaunchKernelGGL((k_graphcut_host<double>), dim3(1), dim3(CB), lds, s, (const double*)dA, (const double*)dB,
+    hipLaunchKernelGGL(cut_host_kernel<double>(npt), dim3(1), dim3(team), lds, s, (const double*)dA, (const double*)dB,
                        s0, s1, s2, dim, keep, gscr, err);
   HCL();
 }
@@ -2982,7 +3000,7 @@ int iq_graphcut(iq_ctx* ctx, const void* A, const void* B, int dtype, const int6
     uint8_t* keep = m.alloc<uint8_t>(nvox);
     int32_t* err = m.alloc<int32_t>(1);
     HC(hipMemsetAsync(err, 0, sizeof(int32_t), s));
-    char* gscr = n > IQ_PR_NLDS ? m.alloc<char>((size_t)n * CUT_NODE_BYTES) : nullptr;
+    char* gscr = n > CUT_REG_MAX ? m.alloc<char>((size_t)n * CUT_NODE_BYTES) : nullptr;
     cut_launch(s, dA, dB, dtype, dims, dim, n, keep, gscr, err);
     int32_t code = 0;
     HC(hipMemcpyAsync(&code, err, sizeof(int32_t), hipMemcpyDeviceToHost, s));
@@ -3003,7 +3021,7 @@ int iq_graphcut_noalloc(iq_ctx* ctx, const void* A, const void* B, int dtype, co
                                   std::to_string(IQ_NOALLOC_MAX_NODES));
     char* base = scratch_ptr(ctx->device);
     int32_t* err = (int32_t*)base;
-    char* gscr = n > IQ_PR_NLDS ? base + IQ_NOALLOC_HEAD : nullptr;
+    char* gscr = n > CUT_REG_MAX ? base + IQ_NOALLOC_HEAD : nullptr;
     hipStream_t s = ctx->stream;
     // the status word keeps the previous call's value: cleared by a kernel
     hipLaunchKernelGGL((k_fill<int32_t>), dim3(1), dim3(64), 0, s, err, (int64_t)1, (int32_t)0);

@@ -15,7 +15,6 @@
 #define IQ_GR_BIG 1024
 #define IQ_PR_LIMIT 200000  // push-relabel round guard (never reached on valid input)
 #define IQ_SORT_MAX 4096    // largest multi-valued band ranked in LDS
-#define IQ_PR_NLDS 1536     // interior min-cut nodes kept in LDS (above: global scratch)
 
 // error codes written by kernels into the per-run flag word (first error wins)
 #define IQ_KERR_NOCAND 1

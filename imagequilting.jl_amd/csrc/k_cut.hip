@@ -1,10 +1,10 @@
 // k_cut.hip -- boundary cut (graphcut.jl:5-84) and paste (iqsim.jl:252-281).
 //
-// One 256-wide workgroup per overlap slab.  The first slice along the cut
+// One workgroup per overlap slab.  The first slice along the cut
 // axis is tied to the source and the last to the sink with infinite capacity
 // (graphcut.jl:56-70), so both are contracted into the terminals and a
-// preflow push-relabel runs on the interior slices, its state resident in LDS
-// (global scratch beyond IQ_PR_NLDS interior nodes).  The schedule is
+// preflow push-relabel runs on the interior slices, its state in registers and
+// LDS (global scratch beyond CUT_REG_MAX interior nodes).  The schedule is
 // synchronous: a relabel phase, a push phase (only the higher endpoint of an
 // edge can push on it, so every residual pair has one writer) and a gather
 // phase that adds incoming flow in a fixed neighbour order; a global relabel
@@ -13,8 +13,6 @@
 // restatement bit for bit.  Cut mask = voxels that cannot reach the sink in
 // the residual graph (graphcut.jl:79-81).
 #include "iq_internal.h"
-
-#define CB 256
 
 template <typename T>
 __device__ inline double cut_cap(const T* A, const T* B, int64_t u, int64_t v, int64_t w, bool wok);
@@ -90,14 +88,15 @@ __device__ inline void cut_bind(CutState& S, char* mem, int n) {
 // Minimum cut of one slab (graphcut.jl:5-84) by the whole workgroup: writes
 // keep = mask XOR side for every slab voxel into out (slab column-major).
 // A and B are strided views (the simulation grid and the chosen training-image
-// window); S points at LDS or global scratch sized for the interior nodes.
+// window); S points at global scratch sized for the interior nodes.
 template <typename T>
 __device__ void cut_slab(const SlabView<T>& A, const SlabView<T>& B, const int s[3], int dim, uint8_t side,
                          uint8_t* out, char* mem, int32_t* err, int64_t* rounds) {
+  const int TEAM = (int)blockDim.x;
   const int L = s[dim];
   const int nvox = s[0] * s[1] * s[2];
   // terminal slices
-  for (int p = threadIdx.x; p < nvox; p += CB) {
+  for (int p = threadIdx.x; p < nvox; p += TEAM) {
     int c[3] = {p % s[0], (p / s[0]) % s[1], p / (s[0] * s[1])};
     uint8_t m = (c[dim] == L - 1) ? 0 : 1;
     out[p] = m ^ side;
@@ -113,7 +112,7 @@ __device__ void cut_slab(const SlabView<T>& A, const SlabView<T>& B, const int s
   cut_bind(S, mem, n);
 
   // build: capacities of graphcut.jl:22-54 on interior edges; saturated source edges
-  for (int u = threadIdx.x; u < n; u += CB) {
+  for (int u = threadIdx.x; u < n; u += TEAM) {
     int ic[3] = {u % si[0], (u / si[0]) % si[1], u / (si[0] * si[1])};
     int pc[3] = {ic[0], ic[1], ic[2]};
     pc[dim] += 1;
@@ -141,11 +140,11 @@ __device__ void cut_slab(const SlabView<T>& A, const SlabView<T>& B, const int s
   int64_t total = 0;
   for (;;) {
     // global relabel
-    for (int u = threadIdx.x; u < n; u += CB) S.h[u] = ((S.fl[u] & 8) && S.rt[u] > 0.0) ? 1 : HMAX;
+    for (int u = threadIdx.x; u < n; u += TEAM) S.h[u] = ((S.fl[u] & 8) && S.rt[u] > 0.0) ? 1 : HMAX;
     __syncthreads();
     for (int lev = 1;; lev++) {
       int ch = 0;
-      for (int u = threadIdx.x; u < n; u += CB) {
+      for (int u = threadIdx.x; u < n; u += TEAM) {
         if (S.h[u] != HMAX) continue;
         int ic[3] = {u % si[0], (u / si[0]) % si[1], u / (si[0] * si[1])};
         bool hit = false;
@@ -164,7 +163,7 @@ __device__ void cut_slab(const SlabView<T>& A, const SlabView<T>& B, const int s
       if (!__syncthreads_or(ch)) break;
     }
     int act = 0;
-    for (int u = threadIdx.x; u < n; u += CB) act |= (S.e[u] > 0.0 && S.h[u] < HMAX);
+    for (int u = threadIdx.x; u < n; u += TEAM) act |= (S.e[u] > 0.0 && S.h[u] < HMAX);
     if (!__syncthreads_or(act)) break;
     if (total > IQ_PR_LIMIT) {
       if (threadIdx.x == 0) atomicCAS(err, 0, IQ_KERR_ITER);
@@ -172,7 +171,7 @@ __device__ void cut_slab(const SlabView<T>& A, const SlabView<T>& B, const int s
     }
     for (int it = 0; it < GR; it++) {
       // relabel phase (also clears the push records of the previous round)
-      for (int u = threadIdx.x; u < n; u += CB) {
+      for (int u = threadIdx.x; u < n; u += TEAM) {
         S.pr[3 * u] = 0.0; S.pr[3 * u + 1] = 0.0; S.pr[3 * u + 2] = 0.0;
         int hu = S.h[u];
         int nh = hu;
@@ -196,10 +195,10 @@ __device__ void cut_slab(const SlabView<T>& A, const SlabView<T>& B, const int s
         S.hn[u] = nh;
       }
       __syncthreads();
-      for (int u = threadIdx.x; u < n; u += CB) S.h[u] = S.hn[u];
+      for (int u = threadIdx.x; u < n; u += TEAM) S.h[u] = S.hn[u];
       __syncthreads();
       // push phase
-      for (int u = threadIdx.x; u < n; u += CB) {
+      for (int u = threadIdx.x; u < n; u += TEAM) {
         double ex = S.e[u];
         int hu = S.h[u];
         if (!(ex > 0.0 && hu < HMAX)) continue;
@@ -243,7 +242,7 @@ __device__ void cut_slab(const SlabView<T>& A, const SlabView<T>& B, const int s
       __syncthreads();
       // gather phase
       int a2 = 0;
-      for (int u = threadIdx.x; u < n; u += CB) {
+      for (int u = threadIdx.x; u < n; u += TEAM) {
         int ic[3] = {u % si[0], (u / si[0]) % si[1], u / (si[0] * si[1])};
         double ex = S.e[u];
         for (int d = 0; d < 3; d++) {
@@ -263,7 +262,7 @@ __device__ void cut_slab(const SlabView<T>& A, const SlabView<T>& B, const int s
       if (!__syncthreads_or(a2)) break;
     }
   }
-  for (int u = threadIdx.x; u < n; u += CB) {
+  for (int u = threadIdx.x; u < n; u += TEAM) {
     int ic[3] = {u % si[0], (u / si[0]) % si[1], u / (si[0] * si[1])};
     int pc[3] = {ic[0], ic[1], ic[2]};
     pc[dim] += 1;
@@ -276,26 +275,44 @@ __device__ void cut_slab(const SlabView<T>& A, const SlabView<T>& B, const int s
   }
 }
 
-// Register-resident form of cut_slab for slabs of at most NPT * TEAM
-// interior nodes: same schedule, same arithmetic, bit-identical result.  A
-// work-item owns nodes u = tid + k * TEAM; their coordinates, excess, sink
-// residual, flags, height and the residuals of their six outgoing edges
-// (towards the minus and the plus neighbour per axis) stay in registers:
-// only the owner reads them.  A push from u to w lowers u's outgoing
-// residual at once and leaves the amount in w's inbox (LDS, one slot per
-// direction a push can come from, so each slot has one writer); w adds it
-// to its excess and to its own outgoing residual on that edge at the start
-// of the next round, in the same fixed order as the reference schedule's
-// gather.  LDS holds only the inboxes (6 doubles per node) and the heights
-// (double buffered, 16-bit): 52 bytes per node, so a 1,536-node slab takes
-// 78 KB and two slabs fit in one compute unit.  A round costs two barriers.
-// Team synchronisation of the register-resident cut: a 64-wide team is one
-// wavefront (its LDS accesses complete in order; the fences only stop the
-// compiler from moving them across the step), wider teams use the
-// workgroup barrier.
-template <int TEAM>
-__device__ inline void team_sync() {
-  if constexpr (TEAM == 64) {
+// Register-resident form of cut_slab: same schedule, same arithmetic,
+// bit-identical result.  A work-item owns nodes u = tid + k * TEAM, k < NPT;
+// their excess, sink residual, height and the residuals of their six outgoing
+// edges (towards the minus and the plus neighbour per axis; zero where the
+// edge is absent) stay in registers: only the owner reads them.  A push from u
+// to w lowers u's outgoing residual at once and leaves the amount in w's inbox
+// (LDS, one slot per direction a push can come from, so each slot has one
+// writer); w adds it to its excess and to its own outgoing residual on that
+// edge at the start of the next round, in the same fixed order as the
+// reference schedule's gather.  LDS holds only the inboxes (6 doubles per
+// node) and the heights (double buffered, 16-bit): 52 bytes per node.
+//
+// A round is two barriers around straight-line code: with one node a lane its
+// time is the length of that instruction stream (one wavefront per SIMD), with
+// six node-wavefronts per SIMD (1,536 nodes) its issue slots, so what the
+// schedule allows is done without branches, tests and clears:
+//   * a wavefront with excess rewrites all six outgoing amounts of its nodes,
+//     zeros included, so a received amount needs no test (adding zero changes
+//     nothing) and no clearing; it writes zeros once more in the first round
+//     without excess, then skips the push altogether.  The slot of an absent
+//     edge is the node's own inbox slot that no neighbour writes;
+//   * heights are valid labels (h(u) <= h(v) + 1 on every residual edge u->v:
+//     relabels take a minimum over neighbours that only rise, and a push opens
+//     an edge from the lower to the higher end), so an active node's relabel,
+//     with or without an admissible edge, is min over residual edges of
+//     h(v) + 1;
+//   * neighbour indices and inbox addresses are formed once per slab.
+// 96 slabs side by side, with tests, branches and clears and now: 200 nodes on
+// 256 lanes 129 and 87 us, 576 nodes on 256 lanes with three each 455 us and on
+// 576 lanes 152 us, 1,536 nodes 741 and 489 us.  The node state must start on a
+// 16-byte boundary: 8-byte LDS accesses that straddle one run ten times slower.
+//
+// OR of a predicate over the team: wavefront votes into one of three LDS words
+// behind a single barrier; the word used next is cleared before the barrier
+// (its last readers passed an earlier one).
+template <bool WAVE>
+__device__ __forceinline__ void team_sync() {
+  if constexpr (WAVE) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -304,32 +321,69 @@ __device__ inline void team_sync() {
   }
 }
 
-// OR of a predicate over the team: wavefront ballots, then (wider teams)
-// one flag per wavefront in LDS behind a single barrier; the flags alternate
-// between two buffers so the next call cannot overwrite a flag still unread.
-template <int TEAM>
-__device__ inline bool team_or(int p, int* tflag, int& par) {
-  if constexpr (TEAM == 64) {
-    team_sync<64>();
-    return __any(p);
+template <bool WAVE>
+__device__ __forceinline__ bool team_or(bool p, int* tflag, int& ph) {
+  const bool w = __any(p);
+  if constexpr (WAVE) {
+    team_sync<true>();
+    return w;
   } else {
-    const bool w = __any(p);
-    int* f = tflag + par * (TEAM / 64);
-    if ((threadIdx.x & 63) == 0) f[threadIdx.x >> 6] = w ? 1 : 0;
+    const int nx = ph == 2 ? 0 : ph + 1;
+    if (w && (threadIdx.x & 63) == 0) tflag[ph] = 1;
+    if (threadIdx.x == 0) tflag[nx] = 0;
     __syncthreads();
-    int r = 0;
-#pragma unroll
-    for (int i = 0; i < TEAM / 64; i++) r |= f[i];
-    par ^= 1;
+    const int r = __builtin_amdgcn_readfirstlane(tflag[ph]);
+    ph = nx;
     return r != 0;
   }
 }
 
-#define CUT_FAST_NODE_BYTES (8 * 6 + 2 * 2)
+// The same in two parts: the vote and its barrier, returning the word to read;
+// the word itself, to be tested (readfirstlane) before the next barrier.
+template <bool WAVE>
+__device__ __forceinline__ int team_vote(bool p, int* tflag, int& ph) {
+  if constexpr (WAVE) {
+    team_sync<true>();
+    return 0;
+  } else {
+    const int cur = ph, nx = ph == 2 ? 0 : ph + 1;
+    if (p) tflag[cur] = 1;
+    if (threadIdx.x == 0) tflag[nx] = 0;
+    __syncthreads();
+    ph = nx;
+    return cur;
+  }
+}
+template <bool WAVE>
+__device__ __forceinline__ int team_votes(bool p, const int* tflag, int cur) {
+  if constexpr (WAVE) return __any(p);
+  else return tflag[cur];
+}
 
-template <typename T, int NPT, int TEAM>
+// max(x, 0) with zero for NaN (infinite less infinite), and the lesser of two
+// numbers: one instruction each (the compiler's own forms quiet their operands
+// first, which no value here needs).
+__device__ __forceinline__ double cut_pos(double x) {
+  double y;
+  asm("v_max_f64 %0, %1, 0" : "=v"(y) : "v"(x));
+  return y;
+}
+__device__ __forceinline__ double cut_min(double x, double z) {
+  double y;
+  asm("v_min_f64 %0, %1, %2" : "=v"(y) : "v"(x), "v"(z));
+  return y;
+}
+
+#define CUT_FAST_NODE_BYTES (8 * 6 + 2 * 2)
+#define CUT_TEAM_MAX 1024
+#define CUT_REG_MAX (3 * CUT_TEAM_MAX)  // nodes of the register-resident form (159,744 bytes of LDS)
+
+// mem: CUT_FAST_NODE_BYTES for every node, the count rounded up to a multiple
+// of 64; TEAM = 64 (WAVE) or the workgroup's size, a multiple of 64.
+template <typename T, int NPT, bool WAVE, bool SKIP = (NPT > 1)>
 __device__ __forceinline__ void cut_slab_fast(const SlabView<T>& A, const SlabView<T>& B, const int s[3], int dim, uint8_t side,
-                              uint8_t* out, char* mem, int32_t* err, int64_t* rounds) {
+                                              uint8_t* out, char* mem, int32_t* err, int64_t* rounds) {
+  const int TEAM = WAVE ? 64 : (int)blockDim.x;
   const int L = s[dim];
   const int nvox = s[0] * s[1] * s[2];
   for (int p = threadIdx.x; p < nvox; p += TEAM) {
@@ -341,241 +395,248 @@ __device__ __forceinline__ void cut_slab_fast(const SlabView<T>& A, const SlabVi
   int si[3] = {s[0], s[1], s[2]};
   si[dim] = L - 2;
   const int n = si[0] * si[1] * si[2];
+  const int np = (n + 63) & ~63;
   const int HMAX = n + 1;
   const int GR = iq_gr_freq(n);
   const int ist[3] = {1, si[0], si[0] * si[1]};
-  __shared__ int tflag[2 * (TEAM / 64)];
-  int par = 0;
-  // inbox of node w: [6 w + d] the amount its minus neighbour along d pushed
-  // up to it, [6 w + 3 + d] what its plus neighbour pushed down
+  __shared__ int tflag[3];
+  int ph = 0;
+  // inbox of node w: [d np + w] the amount its minus neighbour along d pushed
+  // up to it, [(3 + d) np + w] what its plus neighbour pushed down
   double* inb = (double*)mem;
-  int16_t* h = (int16_t*)(inb + 6 * n);  // committed heights
-  int16_t* hn = h + n;                   // next heights
-  // per owned node: flags (bit d: plus edge d, bit 3: sink edge, bits 4+d: minus edge d),
-  // excess, sink residual, outgoing residuals towards the minus (om) and plus
-  // (op) neighbours, height; neighbour indices are formed where used
-  // (clamped to the node itself where the edge is absent)
-  int fl[NPT];
-  int uu[NPT];
+  int16_t* h = (int16_t*)(inb + 6 * np);  // committed heights
+  int16_t* hn = h + np;                   // next heights
+  // per owned node: excess, sink residual, outgoing residuals towards the
+  // minus (om) and plus (op) neighbours, height; neighbour indices (the node
+  // itself where the edge is absent) and the inbox slots its pushes go to
+  bool live[NPT];  // uniform per wavefront: it holds nodes (its lanes past n hold isolated ones)
   double e[NPT], rt[NPT], om[NPT][3], op[NPT][3];
-  int hr[NPT];
-#define CUT_VM(k, d) ((fl[k] & (16 << (d))) ? uu[k] - ist[d] : uu[k])
-#define CUT_VP(k, d) ((fl[k] & (1 << (d))) ? uu[k] + ist[d] : uu[k])
+  int hr[NPT], vm[NPT][3], vp[NPT][3], qm[NPT][3], qp[NPT][3];
+  bool dirty[NPT];  // uniform per wavefront: it wrote a nonzero amount last round
 #pragma unroll
   for (int k = 0; k < NPT; k++) {
     const int u = threadIdx.x + k * TEAM;
-    uu[k] = u;
-    fl[k] = 0;
+    live[k] = (int)(threadIdx.x & ~63u) + k * TEAM < n;
+    dirty[k] = false;
     e[k] = 0.0;
     rt[k] = 0.0;
     hr[k] = HMAX;
-#pragma unroll
+    int ic[3] = {u % si[0], (u / si[0]) % si[1], u / (si[0] * si[1])};
+    int pc[3] = {ic[0], ic[1], ic[2]};
+    pc[dim] += 1;
     for (int d = 0; d < 3; d++) {
       om[k][d] = 0.0;
       op[k][d] = 0.0;
+      vm[k][d] = u;
+      vp[k][d] = u;
+      qm[k][d] = d * np + u;
+      qp[k][d] = (3 + d) * np + u;
+      if (u >= n) continue;
+      // an edge's capacity is the same both ways; each end evaluates it
+      if (ic[d] + 1 < si[d]) {
+        op[k][d] = slab_cap<T>(A, B, s, pc[0], pc[1], pc[2], d);
+        vp[k][d] = u + ist[d];
+        qp[k][d] = d * np + u + ist[d];
+      }
+      if (ic[d] > 0) {
+        int q[3] = {pc[0], pc[1], pc[2]};
+        q[d] -= 1;
+        om[k][d] = slab_cap<T>(A, B, s, q[0], q[1], q[2], d);
+        vm[k][d] = u - ist[d];
+        qm[k][d] = (3 + d) * np + u - ist[d];
+      }
     }
     if (u < n) {
-      int ic[3] = {u % si[0], (u / si[0]) % si[1], u / (si[0] * si[1])};
-      int pc[3] = {ic[0], ic[1], ic[2]};
-      pc[dim] += 1;
-      int f = 0;
-      for (int d = 0; d < 3; d++) {
-        // an edge's capacity is the same both ways; each end evaluates it
-        if (ic[d] + 1 < si[d]) { f |= 1 << d; op[k][d] = slab_cap<T>(A, B, s, pc[0], pc[1], pc[2], d); }
-        if (ic[d] > 0) {
-          int q[3] = {pc[0], pc[1], pc[2]};
-          q[d] -= 1;
-          f |= 16 << d;
-          om[k][d] = slab_cap<T>(A, B, s, q[0], q[1], q[2], d);
-        }
-        inb[6 * u + d] = 0.0;
-        inb[6 * u + 3 + d] = 0.0;
-      }
       if (pc[dim] == 1) {
         int q[3] = {pc[0], pc[1], pc[2]};
         q[dim] -= 1;
         e[k] = e[k] + slab_cap<T>(A, B, s, q[0], q[1], q[2], dim);
       }
-      if (pc[dim] == L - 2) { f |= 8; rt[k] = slab_cap<T>(A, B, s, pc[0], pc[1], pc[2], dim); }
-      fl[k] = f;
+      if (pc[dim] == L - 2) rt[k] = slab_cap<T>(A, B, s, pc[0], pc[1], pc[2], dim);
+    }
+    if (live[k]) {
+#pragma unroll
+      for (int d = 0; d < 6; d++) inb[d * np + u] = 0.0;
     }
   }
-  team_sync<TEAM>();
+  if (threadIdx.x < 3) tflag[threadIdx.x] = 0;
+  team_sync<WAVE>();
 
   int64_t total = 0, levels = 0;
   for (;;) {
-    // global relabel (exact residual distance to the sink)
+    // global relabel (exact residual distance to the sink): the least fixed
+    // point of h(u) = min over residual edges u->v of h(v) + 1 from these
+    // starting values, which relaxing in any order reaches as well as a
+    // level-by-level BFS does (every label written is the length of a real
+    // path, and labels only decrease).
 #pragma unroll
     for (int k = 0; k < NPT; k++)
-      if (uu[k] < n) h[uu[k]] = (int16_t)(((fl[k] & 8) && rt[k] > 0.0) ? 1 : HMAX);
-    team_sync<TEAM>();
-    // The labels are the residual hop distances to the sink (+1): the least
-    // fixed point of h(u) = min over residual edges u->v of h(v) + 1 from
-    // these starting values, which relaxing in any order reaches as well as
-    // a level-by-level BFS does (every label written is the length of a real
-    // path, and labels only decrease).
+      if (live[k]) {
+        hr[k] = rt[k] > 0.0 ? 1 : HMAX;
+        h[threadIdx.x + k * TEAM] = (int16_t)hr[k];
+      }
+    team_sync<WAVE>();
+    int rm[NPT][3], rp[NPT][3];  // the neighbour, or the node itself where the edge is saturated
+#pragma unroll
+    for (int k = 0; k < NPT; k++)
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        const int u = threadIdx.x + k * TEAM;
+        rm[k][d] = om[k][d] > 0.0 ? vm[k][d] : u;
+        rp[k][d] = op[k][d] > 0.0 ? vp[k][d] : u;
+      }
     for (;;) {
       // Each wavefront relaxes its own nodes until they hold still (no
       // barrier; labels of other wavefronts' nodes read meanwhile are valid
       // upper bounds), then one team OR asks whether any wavefront lowered a
       // label; a pass in which none did ends the relabel.  Labels strictly
       // decrease, so both loops end.
-      int ch = 0;
+      bool ch = false;
       for (;;) {
-        int lc = 0;
+        bool lc = false;
 #pragma unroll
-        for (int k = 0; k < NPT; k++) {
-          const int u = uu[k];
-          if (u >= n) continue;
-          const int hu = h[u];
-          int hm[3], hp[3];
+        for (int r = 0; r < 2; r++) {
 #pragma unroll
-          for (int d = 0; d < 3; d++) { hm[d] = h[CUT_VM(k, d)]; hp[d] = h[CUT_VP(k, d)]; }
-          int best = hu;
-#pragma unroll
-          for (int d = 0; d < 3; d++) {
-            if ((fl[k] & (16 << d)) && om[k][d] > 0.0 && hm[d] + 1 < best) best = hm[d] + 1;
-            if ((fl[k] & (1 << d)) && op[k][d] > 0.0 && hp[d] + 1 < best) best = hp[d] + 1;
+          for (int k = 0; k < NPT; k++) {
+            if (!live[k]) continue;
+            const int u = threadIdx.x + k * TEAM;
+            const int hu = hr[k];
+            const int a0 = h[rm[k][0]], a1 = h[rm[k][1]], a2 = h[rm[k][2]];
+            const int b0 = h[rp[k][0]], b1 = h[rp[k][1]], b2 = h[rp[k][2]];
+            const int best = min(min(min(a0, a1), min(a2, b0)), min(b1, b2)) + 1;
+            hr[k] = min(best, hu);
+            h[u] = (int16_t)hr[k];
+            lc |= best < hu;
           }
-          if (best < hu) { h[u] = (int16_t)best; lc = 1; }
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
         if (!__any(lc)) break;
-        ch = 1;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        ch = true;
       }
       levels++;
-      if (!team_or<TEAM>(ch, tflag, par)) break;
+      if (!team_or<WAVE>(ch, tflag, ph)) break;
     }
-    int act = 0;
+    bool act = false;
 #pragma unroll
     for (int k = 0; k < NPT; k++)
-      if (uu[k] < n) {
-        hr[k] = h[uu[k]];
-        act |= (e[k] > 0.0 && hr[k] < HMAX);
-      }
-    if (!team_or<TEAM>(act, tflag, par)) break;
+      if (live[k]) act |= e[k] > 0.0 && hr[k] < HMAX;
+    if (!team_or<WAVE>(act, tflag, ph)) break;
     if (total > IQ_PR_LIMIT) {
       if (threadIdx.x == 0) atomicCAS(err, 0, IQ_KERR_ITER);
       break;
     }
     for (int it = 0; it <= GR; it++) {
       // phase A: take in the previous round's pushes, then relabel
-      int a2 = 0;
-      int hnx[NPT];
+      int hu[NPT];  // the height a push goes to, or -2
+      bool any[NPT];
+      bool a2 = false;
 #pragma unroll
       for (int k = 0; k < NPT; k++) {
-        const int u = uu[k];
-        hnx[k] = hr[k];
-        if (u >= n) continue;
-        const int hu = hr[k];
+        const int u = threadIdx.x + k * TEAM;
+        any[k] = false;
+        hu[k] = -2;
+        if (!live[k]) continue;
+        int hm[3], hp[3];
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+          hm[d] = h[vm[k][d]];
+          hp[d] = h[vp[k][d]];
+        }
         if (it > 0) {
           double im[3], ip[3];
 #pragma unroll
           for (int d = 0; d < 3; d++) {
-            im[d] = inb[6 * u + d];
-            ip[d] = inb[6 * u + 3 + d];
+            im[d] = inb[d * np + u];
+            ip[d] = inb[(3 + d) * np + u];
           }
           double ex = e[k];
 #pragma unroll
           for (int d = 0; d < 3; d++) {
-            if ((fl[k] & (16 << d)) && im[d] > 0.0) {
-              ex += im[d];
-              om[k][d] = om[k][d] + im[d];
-              inb[6 * u + d] = 0.0;
-            }
-            if ((fl[k] & (1 << d)) && ip[d] > 0.0) {
-              ex += ip[d];
-              op[k][d] = op[k][d] + ip[d];
-              inb[6 * u + 3 + d] = 0.0;
-            }
+            ex += im[d];
+            om[k][d] = om[k][d] + im[d];
+            ex += ip[d];
+            op[k][d] = op[k][d] + ip[d];
           }
           e[k] = ex;
         }
-        int nh = hu;
-        const bool active = e[k] > 0.0 && hu < HMAX;
+        const bool active = e[k] > 0.0 && hr[k] < HMAX;
         a2 |= active;
-        if (active && it < GR) {
-          int hm[3], hp[3];
-#pragma unroll
-          for (int d = 0; d < 3; d++) {
-            hm[d] = h[CUT_VM(k, d)];
-            hp[d] = h[CUT_VP(k, d)];
-          }
-          bool adm = false;
+        any[k] = !SKIP || __any(active);
+        if (any[k]) {
           int mh = HMAX;
-          if ((fl[k] & 8) && rt[k] > 0.0) { if (hu == 1) adm = true; mh = 0; }
 #pragma unroll
           for (int d = 0; d < 3; d++) {
-            if ((fl[k] & (16 << d)) && om[k][d] > 0.0) { if (hu == hm[d] + 1) adm = true; if (hm[d] < mh) mh = hm[d]; }
-            if ((fl[k] & (1 << d)) && op[k][d] > 0.0) { if (hu == hp[d] + 1) adm = true; if (hp[d] < mh) mh = hp[d]; }
+            mh = min(mh, om[k][d] > 0.0 ? hm[d] : HMAX);
+            mh = min(mh, op[k][d] > 0.0 ? hp[d] : HMAX);
           }
-          if (!adm) nh = (mh + 1 < HMAX) ? mh + 1 : HMAX;
+          mh = rt[k] > 0.0 ? 0 : mh;
+          // past the last round (it == GR) the heights are not used again
+          hr[k] = active ? min(mh + 1, HMAX) : hr[k];
+          hu[k] = active && mh + 1 < HMAX ? mh : -2;
         }
-        hn[u] = (int16_t)nh;
-        hnx[k] = nh;
+        hn[u] = (int16_t)hr[k];
       }
-      if (it > 0) {
-        total++;
-        if (!team_or<TEAM>(a2, tflag, par)) break;
-      } else {
-        team_sync<TEAM>();
-      }
+      total += it > 0;
+      const int cur = team_vote<WAVE>(a2, tflag, ph);
       if (it == GR) break;
+      const int more = team_votes<WAVE>(a2, tflag, cur);  // read below, past the push
       { int16_t* t = h; h = hn; hn = t; }
-#pragma unroll
-      for (int k = 0; k < NPT; k++) hr[k] = hnx[k];
       // phase B: push with the new heights (an edge has one pusher per
       // round, its higher end: the residuals it reads are its own)
 #pragma unroll
       for (int k = 0; k < NPT; k++) {
-        const int u = uu[k];
-        if (u >= n) continue;
-        double ex = e[k];
-        const int hu = hr[k];
-        if (!(ex > 0.0 && hu < HMAX)) continue;
-        int hm[3], hp[3];
+        if (!live[k]) continue;
+        if (any[k]) {
+          int hm[3], hp[3];
 #pragma unroll
-        for (int d = 0; d < 3; d++) {
-          hm[d] = h[CUT_VM(k, d)];
-          hp[d] = h[CUT_VP(k, d)];
-        }
-        if ((fl[k] & 8) && hu == 1 && rt[k] > 0.0) {
-          double r = rt[k];
-          double dl = ex < r ? ex : r;
-          ex -= dl;
-          rt[k] = r - dl;
-        }
+          for (int d = 0; d < 3; d++) {
+            hm[d] = h[vm[k][d]];
+            hp[d] = h[vp[k][d]];
+          }
+          // what each admissible edge can take
+          double cm[3], cp[3];
+          const double ct = cut_pos(hu[k] == 0 ? rt[k] : 0.0);
 #pragma unroll
-        for (int d = 0; d < 3; d++) {
-          if (ex > 0.0 && (fl[k] & (16 << d)) && hu == hm[d] + 1) {
-            double r = om[k][d];
-            if (r > 0.0) {
-              double dl = ex < r ? ex : r;
-              ex -= dl;
-              om[k][d] = r - dl;
-              inb[6 * (u - ist[d]) + 3 + d] = dl;
-            }
+          for (int d = 0; d < 3; d++) {
+            cm[d] = cut_pos(hu[k] == hm[d] ? om[k][d] : 0.0);
+            cp[d] = cut_pos(hu[k] == hp[d] ? op[k][d] : 0.0);
           }
-          if (ex > 0.0 && (fl[k] & (1 << d)) && hu == hp[d] + 1) {
-            double r = op[k][d];
-            if (r > 0.0) {
-              double dl = ex < r ? ex : r;
-              ex -= dl;
-              op[k][d] = r - dl;
-              inb[6 * (u + ist[d]) + d] = dl;
-            }
+          double ex = e[k];
+          const double dt = cut_min(cut_pos(ex), ct);
+          ex -= dt;
+          rt[k] -= dt;
+#pragma unroll
+          for (int d = 0; d < 3; d++) {
+            const double d0 = cut_min(cut_pos(ex), cm[d]);
+            ex -= d0;
+            om[k][d] -= d0;
+            inb[qm[k][d]] = d0;
+            const double d1 = cut_min(cut_pos(ex), cp[d]);
+            ex -= d1;
+            op[k][d] -= d1;
+            inb[qp[k][d]] = d1;
           }
+          e[k] = ex;
+          dirty[k] = true;
+        } else if (dirty[k]) {
+#pragma unroll
+          for (int d = 0; d < 3; d++) {
+            inb[qm[k][d]] = 0.0;
+            inb[qp[k][d]] = 0.0;
+          }
+          dirty[k] = false;
         }
-        e[k] = ex;
       }
-      team_sync<TEAM>();
+      team_sync<WAVE>();
+      // no node was active: the push above changed nothing
+      if (it > 0 && !__builtin_amdgcn_readfirstlane(more)) break;
     }
   }
 #pragma unroll
   for (int k = 0; k < NPT; k++) {
-    const int u = uu[k];
+    const int u = threadIdx.x + k * TEAM;
     if (u >= n) continue;
     int ic[3] = {u % si[0], (u / si[0]) % si[1], u / (si[0] * si[1])};
     int pc[3] = {ic[0], ic[1], ic[2]};
@@ -588,167 +649,127 @@ __device__ __forceinline__ void cut_slab_fast(const SlabView<T>& A, const SlabVi
     atomicAdd((unsigned long long*)rounds + 1, (unsigned long long)levels);
     atomicAdd((unsigned long long*)rounds + 2, 1ull);
   }
-#undef CUT_VM
-#undef CUT_VP
 }
 
-template <typename T>
-__device__ void cut_dispatch(const SlabView<T>& A, const SlabView<T>& B, const int s[3], int dim, uint8_t side,
-                             uint8_t* out, char* lds, char* gmem, int32_t* err, int64_t* rounds) {
+// One slab by the whole workgroup (a multiple of 64 work-items): up to NPT
+// register-resident nodes a lane; NPT = 0: node state in global scratch.
+template <typename T, int NPT>
+__device__ __forceinline__ void cut_dispatch(const SlabView<T>& A, const SlabView<T>& B, const int s[3], int dim, uint8_t side,
+                                             uint8_t* out, char* lds, char* gmem, int32_t* err, int64_t* rounds) {
   const int n = s[0] * s[1] * s[2] / s[dim] * (s[dim] > 2 ? s[dim] - 2 : 0);
-  if (n <= CB) cut_slab_fast<T, 1, CB>(A, B, s, dim, side, out, lds, err, rounds);
-  else if (n <= 2 * CB) cut_slab_fast<T, 2, CB>(A, B, s, dim, side, out, lds, err, rounds);
-  else if (n <= 4 * CB) cut_slab_fast<T, 4, CB>(A, B, s, dim, side, out, lds, err, rounds);
-  else if (n <= IQ_PR_NLDS) cut_slab<T>(A, B, s, dim, side, out, lds, err, rounds);
-  else cut_slab<T>(A, B, s, dim, side, out, gmem, err, rounds);
+  const int team = (int)blockDim.x;
+  if constexpr (NPT == 0) {
+    cut_slab<T>(A, B, s, dim, side, out, gmem, err, rounds);
+  } else {
+    if (NPT >= 3 && n > 2 * team) cut_slab_fast<T, 3, false>(A, B, s, dim, side, out, lds, err, rounds);
+    else if (NPT >= 2 && n > team) cut_slab_fast<T, 2, false>(A, B, s, dim, side, out, lds, err, rounds);
+    else cut_slab_fast<T, 1, false>(A, B, s, dim, side, out, lds, err, rounds);
+  }
 }
 
-
-// Batched cut: grid (slab, query).  A = the realization's grid over the
-// tile, B = the picked training-image window (iqsim.jl:244-273).
+// The slab blockIdx.x of query blockIdx.y: A = the realization's grid over the
+// tile, B = the picked training-image window (iqsim.jl:244-273).  False when
+// there is none.
 template <typename T>
-__global__ void __launch_bounds__(CB)
-k_graphcut(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
-  extern __shared__ char cut_lds[];
+__device__ __forceinline__ bool cut_views(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, SlabView<T>& A,
+                                          SlabView<T>& B, int s[3], int& dim, int& side, uint8_t*& out, char*& gmem) {
   const IqQuery q = qs[blockIdx.y];
   const IqStep& st = D->steps[q.step];
-  if ((int)blockIdx.x >= st.ncut) return;
+  if ((int)blockIdx.x >= st.ncut) return false;
   const int64_t slot = q.slot;
   const int64_t pk = D->pick[slot];
-  if (pk < 0) return;
+  if (pk < 0) return false;
   const IqGeo& g = D->g;
   const IqSlab sl = st.slab[blockIdx.x];
-  const int s[3] = {sl.sz[0], sl.sz[1], sl.sz[2]};
+  for (int d = 0; d < 3; d++) s[d] = sl.sz[d];
+  dim = sl.dim;
+  side = sl.side;
   const int rc[3] = {(int)(pk % g.dist[0]), (int)((pk / g.dist[0]) % g.dist[1]),
                      (int)(pk / ((int64_t)g.dist[0] * g.dist[1]))};
-  SlabView<T> A, B;
   const IqReal& R = D->reals[q.real];
   A.base = (const T*)D->sims + R.sim_off +
            iq_lin3(R.pad, st.origin[0] + sl.lo[0], st.origin[1] + sl.lo[1], st.origin[2] + sl.lo[2]);
   A.st[0] = 1; A.st[1] = R.pad[0]; A.st[2] = (int64_t)R.pad[0] * R.pad[1];
   B.base = (const T*)D->ti + iq_lin3(g.ti, rc[0] + sl.lo[0], rc[1] + sl.lo[1], rc[2] + sl.lo[2]);
   B.st[0] = 1; B.st[1] = g.ti[0]; B.st[2] = (int64_t)g.ti[0] * g.ti[1];
-  uint8_t* out = D->keep + (slot * IQ_MAX_SLAB + blockIdx.x) * g.tilevox;
-  char* gmem = D->cutscratch ? D->cutscratch + (slot * IQ_MAX_SLAB + blockIdx.x) * D->cutscratch_per : nullptr;
-  cut_dispatch<T>(A, B, s, sl.dim, (uint8_t)sl.side, out, cut_lds, gmem, D->err, D->rounds);
+  out = D->keep + (slot * IQ_MAX_SLAB + blockIdx.x) * g.tilevox;
+  gmem = D->cutscratch ? D->cutscratch + (slot * IQ_MAX_SLAB + blockIdx.x) * D->cutscratch_per : nullptr;
+  return true;
 }
 
-template __global__ void k_graphcut<float>(const IqDev*, const IqQuery*);
-template __global__ void k_graphcut<double>(const IqDev*, const IqQuery*);
+// Batched cut: grid (slab, query).  The workgroup has a lane for every node of
+// the plan's largest slab, up to CUT_TEAM_MAX, then two or three nodes a lane.
+template <typename T, int NPT>
+__global__ void __launch_bounds__(CUT_TEAM_MAX)
+k_graphcut(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
+  extern __shared__ __align__(16) char cut_lds[];
+  SlabView<T> A, B;
+  int s[3], dim, side;
+  uint8_t* out;
+  char* gmem;
+  if (!cut_views<T>(D, qs, A, B, s, dim, side, out, gmem)) return;
+  cut_dispatch<T, NPT>(A, B, s, dim, (uint8_t)side, out, cut_lds, gmem, D->err, D->rounds);
+}
+
+#define CUT_INST(T)                                                       \
+  template __global__ void k_graphcut<T, 0>(const IqDev*, const IqQuery*); \
+  template __global__ void k_graphcut<T, 1>(const IqDev*, const IqQuery*); \
+  template __global__ void k_graphcut<T, 2>(const IqDev*, const IqQuery*); \
+  template __global__ void k_graphcut<T, 3>(const IqDev*, const IqQuery*);
+CUT_INST(float)
+CUT_INST(double)
 
 // Plans whose slabs all have at most CUT_WAVE_MAX interior nodes: one
-// wavefront per slab, up to two register-resident nodes per lane, no
-// workgroup barriers in the push-relabel rounds.  (A round costs about the
-// per-node work times the nodes per lane, so beyond two nodes per lane the
-// 256-wide team with one node per lane is faster despite its barriers.)
-#define CUT_WAVE_MAX (2 * 64)
-template <typename T>
-__device__ __forceinline__ void cut_dispatch_wave(const SlabView<T>& A, const SlabView<T>& B, const int s[3], int dim, uint8_t side,
-                                  uint8_t* out, char* lds, int32_t* err, int64_t* rounds) {
-  const int n = s[0] * s[1] * s[2] / s[dim] * (s[dim] > 2 ? s[dim] - 2 : 0);
-  if (n <= 64) cut_slab_fast<T, 1, 64>(A, B, s, dim, side, out, lds, err, rounds);
-  else cut_slab_fast<T, 2, 64>(A, B, s, dim, side, out, lds, err, rounds);
-}
-
+// wavefront per slab, one node a lane, no workgroup barriers in the
+// push-relabel rounds.  (Two nodes a lane cost more than the barriers of twice
+// the lanes: 90-node slabs take 49 us on one wavefront and 34 us on two.)
+#define CUT_WAVE_MAX 64
 template <typename T>
 __global__ void __launch_bounds__(64)
 k_graphcut_wave(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
-  extern __shared__ char cut_lds[];
-  const IqQuery q = qs[blockIdx.y];
-  const IqStep& st = D->steps[q.step];
-  if ((int)blockIdx.x >= st.ncut) return;
-  const int64_t slot = q.slot;
-  const int64_t pk = D->pick[slot];
-  if (pk < 0) return;
-  const IqGeo& g = D->g;
-  const IqSlab sl = st.slab[blockIdx.x];
-  const int s[3] = {sl.sz[0], sl.sz[1], sl.sz[2]};
-  const int rc[3] = {(int)(pk % g.dist[0]), (int)((pk / g.dist[0]) % g.dist[1]),
-                     (int)(pk / ((int64_t)g.dist[0] * g.dist[1]))};
+  extern __shared__ __align__(16) char cut_lds[];
   SlabView<T> A, B;
-  const IqReal& R = D->reals[q.real];
-  A.base = (const T*)D->sims + R.sim_off +
-           iq_lin3(R.pad, st.origin[0] + sl.lo[0], st.origin[1] + sl.lo[1], st.origin[2] + sl.lo[2]);
-  A.st[0] = 1; A.st[1] = R.pad[0]; A.st[2] = (int64_t)R.pad[0] * R.pad[1];
-  B.base = (const T*)D->ti + iq_lin3(g.ti, rc[0] + sl.lo[0], rc[1] + sl.lo[1], rc[2] + sl.lo[2]);
-  B.st[0] = 1; B.st[1] = g.ti[0]; B.st[2] = (int64_t)g.ti[0] * g.ti[1];
-  uint8_t* out = D->keep + (slot * IQ_MAX_SLAB + blockIdx.x) * g.tilevox;
-  cut_dispatch_wave<T>(A, B, s, sl.dim, (uint8_t)sl.side, out, cut_lds, D->err, D->rounds);
+  int s[3], dim, side;
+  uint8_t* out;
+  char* gmem;
+  if (!cut_views<T>(D, qs, A, B, s, dim, side, out, gmem)) return;
+  cut_slab_fast<T, 1, true>(A, B, s, dim, (uint8_t)side, out, cut_lds, D->err, D->rounds);
 }
 
 template __global__ void k_graphcut_wave<float>(const IqDev*, const IqQuery*);
 template __global__ void k_graphcut_wave<double>(const IqDev*, const IqQuery*);
 
-// Plans whose largest slab has CUT_BIG_MIN..CUT_BIG_MAX interior nodes: TEAM
-// (1,024, or 512) work-items per slab, up to two (three) register-resident
-// nodes each (node state of a 1,536-node slab fills the 160 KB of LDS, so one
-// slab per compute unit runs at a time and more lanes per slab shorten each
-// round: config 5's 1,536-node cuts take 1,469 us per launch with 1,024
-// work-items against 1,780 us with 512).
-#define CB_BIG 512
-#define CUT_BIG_MAX 1536
-template <typename T, int TEAM>
-__global__ void __launch_bounds__(TEAM)
-k_graphcut_big(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
-  extern __shared__ char cut_lds[];
-  const IqQuery q = qs[blockIdx.y];
-  const IqStep& st = D->steps[q.step];
-  if ((int)blockIdx.x >= st.ncut) return;
-  const int64_t slot = q.slot;
-  const int64_t pk = D->pick[slot];
-  if (pk < 0) return;
-  const IqGeo& g = D->g;
-  const IqSlab sl = st.slab[blockIdx.x];
-  const int s[3] = {sl.sz[0], sl.sz[1], sl.sz[2]};
-  const int rc[3] = {(int)(pk % g.dist[0]), (int)((pk / g.dist[0]) % g.dist[1]),
-                     (int)(pk / ((int64_t)g.dist[0] * g.dist[1]))};
-  SlabView<T> A, B;
-  const IqReal& R = D->reals[q.real];
-  A.base = (const T*)D->sims + R.sim_off +
-           iq_lin3(R.pad, st.origin[0] + sl.lo[0], st.origin[1] + sl.lo[1], st.origin[2] + sl.lo[2]);
-  A.st[0] = 1; A.st[1] = R.pad[0]; A.st[2] = (int64_t)R.pad[0] * R.pad[1];
-  B.base = (const T*)D->ti + iq_lin3(g.ti, rc[0] + sl.lo[0], rc[1] + sl.lo[1], rc[2] + sl.lo[2]);
-  B.st[0] = 1; B.st[1] = g.ti[0]; B.st[2] = (int64_t)g.ti[0] * g.ti[1];
-  uint8_t* out = D->keep + (slot * IQ_MAX_SLAB + blockIdx.x) * g.tilevox;
-  const int n = s[0] * s[1] * s[2] / s[sl.dim] * (s[sl.dim] > 2 ? s[sl.dim] - 2 : 0);
-  static_assert(3 * TEAM >= CUT_BIG_MAX, "team too small for the largest slab");
-  if (n <= TEAM) cut_slab_fast<T, 1, TEAM>(A, B, s, sl.dim, (uint8_t)sl.side, out, cut_lds, D->err, D->rounds);
-  else if (n <= 2 * TEAM) cut_slab_fast<T, 2, TEAM>(A, B, s, sl.dim, (uint8_t)sl.side, out, cut_lds, D->err, D->rounds);
-  else if constexpr (2 * TEAM < CUT_BIG_MAX)
-    cut_slab_fast<T, 3, TEAM>(A, B, s, sl.dim, (uint8_t)sl.side, out, cut_lds, D->err, D->rounds);
-}
-
-template __global__ void k_graphcut_big<float, 512>(const IqDev*, const IqQuery*);
-template __global__ void k_graphcut_big<double, 512>(const IqDev*, const IqQuery*);
-template __global__ void k_graphcut_big<float, 1024>(const IqDev*, const IqQuery*);
-template __global__ void k_graphcut_big<double, 1024>(const IqDev*, const IqQuery*);
-
 // Standalone cut of one slab pair (iq_graphcut): A and B both column-major of extents s.
-template <typename T>
-__global__ void __launch_bounds__(CB)
+template <typename T, int NPT>
+__global__ void __launch_bounds__(CUT_TEAM_MAX)
 k_graphcut_host(const T* __restrict__ a, const T* __restrict__ b, int s0, int s1, int s2, int dim,
                 uint8_t* __restrict__ out, char* __restrict__ gmem, int32_t* __restrict__ err) {
-  extern __shared__ char cut_lds[];
+  extern __shared__ __align__(16) char cut_lds[];
   const int s[3] = {s0, s1, s2};
   SlabView<T> A, B;
   A.base = a; A.st[0] = 1; A.st[1] = s0; A.st[2] = (int64_t)s0 * s1;
   B.base = b; B.st[0] = 1; B.st[1] = s0; B.st[2] = (int64_t)s0 * s1;
-  cut_dispatch<T>(A, B, s, dim, (uint8_t)0, out, cut_lds, gmem, err, nullptr);
+  cut_dispatch<T, NPT>(A, B, s, dim, (uint8_t)0, out, cut_lds, gmem, err, nullptr);
 }
 
-template __global__ void k_graphcut_host<float>(const float*, const float*, int, int, int, int, uint8_t*, char*, int32_t*);
-template __global__ void k_graphcut_host<double>(const double*, const double*, int, int, int, int, uint8_t*, char*, int32_t*);
+#define CUT_HOST_INST(T)                                                                                         \
+  template __global__ void k_graphcut_host<T, 0>(const T*, const T*, int, int, int, int, uint8_t*, char*, int32_t*); \
+  template __global__ void k_graphcut_host<T, 1>(const T*, const T*, int, int, int, int, uint8_t*, char*, int32_t*); \
+  template __global__ void k_graphcut_host<T, 2>(const T*, const T*, int, int, int, int, uint8_t*, char*, int32_t*); \
+  template __global__ void k_graphcut_host<T, 3>(const T*, const T*, int, int, int, int, uint8_t*, char*, int32_t*);
+CUT_HOST_INST(float)
+CUT_HOST_INST(double)
 
 template <typename T>
 __global__ void __launch_bounds__(64)
 k_graphcut_host_wave(const T* __restrict__ a, const T* __restrict__ b, int s0, int s1, int s2, int dim,
                      uint8_t* __restrict__ out, int32_t* __restrict__ err) {
-  extern __shared__ char cut_lds[];
+  extern __shared__ __align__(16) char cut_lds[];
   const int s[3] = {s0, s1, s2};
   SlabView<T> A, B;
   A.base = a; A.st[0] = 1; A.st[1] = s0; A.st[2] = (int64_t)s0 * s1;
   B.base = b; B.st[0] = 1; B.st[1] = s0; B.st[2] = (int64_t)s0 * s1;
-  cut_dispatch_wave<T>(A, B, s, dim, (uint8_t)0, out, cut_lds, err, nullptr);
+  cut_slab_fast<T, 1, true>(A, B, s, dim, (uint8_t)0, out, cut_lds, err, nullptr);
 }
 
 template __global__ void k_graphcut_host_wave<float>(const float*, const float*, int, int, int, int, uint8_t*, int32_t*);

@@ -114,7 +114,7 @@ int iq_graphcut(iq_ctx* ctx, const void* A, const void* B, int dtype, const int6
  * dims and element type dtype, column-major; out_mask: prod(dims) bytes),
  * their contents ready before the call (the work runs on the context's
  * stream; the call waits for it and returns the cut's status).  The library
- * allocates nothing: the status word and the node state of slabs beyond 1,536
+ * allocates nothing: the status word and the node state of slabs beyond 3,072
  * interior nodes live in one static array per device of
  * 256 + 100 * IQ_NOALLOC_MAX_NODES bytes (about 1.6 MB), held until the
  * process ends.  Slabs with more than IQ_NOALLOC_MAX_NODES interior nodes
