@@ -901,10 +901,14 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
   H.g = g;
   const double* tid = (const double*)d->ti;
   const float* tif = (const float*)d->ti;
+  bool exact16 = false;  // fast, and every value a bf16 (decided on the host's copy: reading the device's costs 1 us a value)
   if (d->ti_dtype == IQ_F32) {
     H.ti = pl->mem.upload(tif, tivox, s);
     pl->fast = fits_range(tif, tivox);
-    if (pl->fast) H.ti32 = (const float*)H.ti;
+    if (pl->fast) {
+      H.ti32 = (const float*)H.ti;
+      exact16 = bf16_exact(tif, tivox);
+    }
   } else {
     H.ti = pl->mem.upload(tid, tivox, s);
     pl->fast = fits_f32(tid, tivox);
@@ -912,6 +916,7 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
     if (pl->fast) {
       std::vector<float> t32((size_t)tivox);
       for (int64_t i = 0; i < tivox; i++) t32[i] = (float)tid[i];
+      exact16 = bf16_exact(t32.data(), tivox);
       H.ti32 = pl->mem.upload(t32.data(), tivox, s);
       HC(hipStreamSynchronize(s));
     }
@@ -1043,7 +1048,7 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
       if (pl->lds_nw[2] || pl->lds_nw[4]) {
         pl->mfma = true;
         pl->mfma_lds = lmax;
-        pl->mfma_split = !bf16_exact(H.ti32, tivox);
+        pl->mfma_split = !exact16;
         pl->mfma_gerr = scan_gerr(H.ktab.nstep, pl->mfma_split, pl->rounded);
         H.chunks = pl->mem.upload(chunks.data(), chunks.size(), s);
         for (int nw : {2, 3, 4}) {
