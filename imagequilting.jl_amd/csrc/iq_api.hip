@@ -251,38 +251,54 @@ bool bf16_exact(const float* v, int64_t n) {
 }
 
 // K table of the MFMA scan over the union of the overlap masks: per box,
-// 8-voxel chunks along x or y (whichever pads less), an even number per box.
+// chunks of cy x (8 / cy) voxels (y by x), whichever of 8, 4 and 2 pads least
+// (the longer one on a tie), an even number per box.  Boxes whose region would
+// take more than SCAN_BOX_LDS are cut along z.
+#define SCAN_BOX_LDS (80 * 1024)
 bool build_ktab(const std::vector<uint8_t>& ubits, const int t3[3], const std::vector<int> brk[3], IqKTab& kt,
                 std::vector<IqChunk>& chunks) {
-  std::vector<IqBox> boxes = decompose(ubits, t3, brk);
+  std::vector<IqBox> boxes;
+  auto shape = [&](const IqBox& b) {
+    int best = 8;
+    int64_t least = INT64_MAX;
+    for (int cy = 8; cy >= 2; cy /= 2) {
+      const int cx = 8 / cy;
+      const int64_t n = (int64_t)((b.wy + cy - 1) / cy) * ((b.wx + cx - 1) / cx);
+      if (n < least) { least = n; best = cy; }
+    }
+    return best;
+  };
+  for (const IqBox& b : decompose(ubits, t3, brk)) {
+    const int cy = shape(b), cx = 8 / cy;
+    const int64_t plane = (int64_t)iq_scan_ry((b.wy + cy - 1) / cy * cy, 4) * iq_scan_rx((b.wx + cx - 1) / cx * cx) * 4;
+    const int parts = (int)std::min<int64_t>(b.wz, (plane * b.wz + SCAN_BOX_LDS - 1) / SCAN_BOX_LDS);
+    for (int p = 0; p < parts; p++) {
+      IqBox c = b;
+      c.z0 = b.z0 + b.wz * p / parts;
+      c.wz = b.z0 + b.wz * (p + 1) / parts - c.z0;
+      boxes.push_back(c);
+    }
+  }
+  if ((int)boxes.size() > IQ_MAX_KBOX) boxes = decompose(ubits, t3, brk);
   if ((int)boxes.size() > IQ_MAX_KBOX) return false;
   kt.nbox = 0;
   int step = 0;
   for (const IqBox& b : boxes) {
-    auto r8 = [](int w) { return (w + 7) / 8 * 8; };
-    const double ex = (double)b.wx / r8(b.wx), ey = (double)b.wy / r8(b.wy);
-    const int dir = (ey > ex) ? 1 : 0;
+    const int cy = shape(b), cx = 8 / cy;
     IqKBox kb{};
     kb.x0 = b.x0; kb.y0 = b.y0; kb.z0 = b.z0; kb.wz = b.wz;
-    kb.wxr = dir == 0 ? r8(b.wx) : b.wx;
-    kb.wyr = dir == 1 ? r8(b.wy) : b.wy;
+    kb.wxr = (b.wx + cx - 1) / cx * cx;
+    kb.wyr = (b.wy + cy - 1) / cy * cy;
+    kb.cy = cy;
     const size_t c0 = chunks.size();
-    for (int z = 0; z < b.wz; z++) {
-      if (dir == 0) {
-        for (int y = 0; y < b.wy; y++)
-          for (int x = 0; x < b.wx; x += 8)
-            chunks.push_back(IqChunk{(int16_t)(b.x0 + x), (int16_t)(b.y0 + y), (int16_t)(b.z0 + z), 0,
-                                     (int8_t)std::min(8, b.wx - x)});
-      } else {
-        for (int x = 0; x < b.wx; x++)
-          for (int y = 0; y < b.wy; y += 8)
-            chunks.push_back(IqChunk{(int16_t)(b.x0 + x), (int16_t)(b.y0 + y), (int16_t)(b.z0 + z), 1,
-                                     (int8_t)std::min(8, b.wy - y)});
-      }
-    }
+    for (int z = 0; z < b.wz; z++)
+      for (int x = 0; x < b.wx; x += cx)
+        for (int y = 0; y < b.wy; y += cy)
+          chunks.push_back(IqChunk{(int16_t)(b.x0 + x), (int16_t)(b.y0 + y), (int16_t)(b.z0 + z), (int8_t)cy,
+                                   (int8_t)std::min(cy, b.wy - y), (int8_t)std::min(cx, b.wx - x)});
     if ((chunks.size() - c0) % 2) {  // zero chunk: same base, no voxels
       IqChunk z = chunks.back();
-      z.n = 0;
+      z.ny = z.nx = 0;
       chunks.push_back(z);
     }
     kb.s0 = step;
@@ -515,6 +531,19 @@ std::vector<std::vector<int64_t>> build_waves(const HostGrid& G, const IqStep* s
   return waves;
 }
 
+// One MFMA scan of nq queries (B fragments prepared) with groups of nw wavefronts.
+dim3 scan_grid(const iq_plan* pl, int nq, int nw) {
+  const IqGeo& g = pl->geo;
+  const int ntile = (nq + 31) / 32;
+  return dim3(nblk(g.dist[0], 32), nblk(g.dist[1], 4 * nw), (unsigned)(g.dist[2] * ntile));
+}
+void launch_scan_mfma(iq_plan* pl, const IqQuery* q, int nq, int nw, hipStream_t s) {
+  hipLaunchKernelGGL((pl->mfma_split ? k_scan_mfma<true> : k_scan_mfma<false>),
+                     scan_grid(pl, nq, nw), dim3(64 * nw), pl->lds_nw[nw], s, (const IqDev*)pl->dd, q, nq, pl->mfma_gerr,
+                     pl->kofs_nw[nw]);
+  HCL();
+}
+
 // Scan autotuner: the MFMA scan's group size (2 or 4 wavefronts) is measured
 // on the plan itself.  A batch of the plan's own masked steps (32 queries,
 // then up to 64 as the slots allow) is prepared once; each group size runs one
@@ -560,17 +589,10 @@ void tune_scan(iq_plan* pl) {
     HCL();
     float best = 1e30f;
     for (int nw : nwa) {
-      dim3 grid(nblk(g.dist[0], 32), nblk(g.dist[1], 4 * nw), (unsigned)(g.dist[2] * ntile));
       float tot = 0.0f;
       for (int rep = 0; rep < 4; rep++) {
         if (rep == 1) HC(hipEventRecord(a, s));
-        if (pl->mfma_split)
-          hipLaunchKernelGGL((k_scan_mfma<true>), grid, dim3(64 * nw), pl->lds_nw[nw], s, D, dq, nq, pl->mfma_gerr,
-                             pl->kofs_nw[nw]);
-        else
-          hipLaunchKernelGGL((k_scan_mfma<false>), grid, dim3(64 * nw), pl->lds_nw[nw], s, D, dq, nq, pl->mfma_gerr,
-                             pl->kofs_nw[nw]);
-        HCL();
+        launch_scan_mfma(pl, dq, nq, nw, s);
       }
       HC(hipEventRecord(b, s));
       HC(hipEventSynchronize(b));
@@ -1018,6 +1040,7 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
       brk[k].erase(std::remove_if(brk[k].begin(), brk[k].end(), [&](int v) { return v < 0 || v > t3[k]; }), brk[k].end());
     }
     std::vector<IqChunk> chunks;
+    const bool split = !exact16;
     if (want && pl->fast && !hmasks.empty() && build_ktab(ubits, t3, brk, H.ktab, chunks)) {
       // Group size: a group of nw wavefronts covers 4 nw candidate rows.
       // Launches of at most about four 4-wavefront groups per compute unit
@@ -1029,7 +1052,7 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
         size_t l = 0;
         for (int b = 0; b < H.ktab.nbox; b++) {
           const IqKBox& kb = H.ktab.box[b];
-          l = std::max(l, (size_t)(32 + kb.wxr - 1) * (4 * nw + kb.wyr - 1) * kb.wz * 4);
+          l = std::max(l, (size_t)iq_scan_rx(kb.wxr) * iq_scan_ry(kb.wyr, nw) * kb.wz * 4);
         }
         return l;
       };
@@ -1045,10 +1068,25 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
         pl->lds_nw[nw] = lds_of(nw);
         lmax = std::max(lmax, pl->lds_nw[nw]);
       }
-      if (pl->lds_nw[2] || pl->lds_nw[4]) {
+      // words past the image that a staged region may cover
+      int rxm = 0, rym = 0;
+      for (int b = 0; b < H.ktab.nbox; b++) {
+        rxm = std::max(rxm, iq_scan_rx(H.ktab.box[b].wxr));
+        rym = std::max(rym, iq_scan_ry(H.ktab.box[b].wyr, 4));
+      }
+      const int64_t nwords = tivox + (int64_t)g.ti[1] * (rxm + 33) + rym + 64;
+      if ((pl->lds_nw[2] || pl->lds_nw[4]) && nwords < (1ll << 31)) {
         pl->mfma = true;
         pl->mfma_lds = lmax;
-        pl->mfma_split = !exact16;
+        pl->mfma_split = split;
+        uint32_t* tiw = pl->mem.alloc<uint32_t>((size_t)nwords);
+        const unsigned pb = (unsigned)std::min<int64_t>(nblk(nwords, 256), 4096);
+        if (split)
+          hipLaunchKernelGGL((k_scan_pack<true>), dim3(pb), dim3(256), 0, s, H.ti32, g.ti[0], g.ti[1], g.ti[2], tiw, nwords);
+        else
+          hipLaunchKernelGGL((k_scan_pack<false>), dim3(pb), dim3(256), 0, s, H.ti32, g.ti[0], g.ti[1], g.ti[2], tiw, nwords);
+        HCL();
+        H.tiw = tiw;
         pl->mfma_gerr = scan_gerr(H.ktab.nstep, pl->mfma_split, pl->rounded);
         H.chunks = pl->mem.upload(chunks.data(), chunks.size(), s);
         for (int nw : {2, 3, 4}) {
@@ -1056,12 +1094,10 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
           std::vector<int32_t> kofs(chunks.size());
           for (int b = 0; b < H.ktab.nbox; b++) {
             const IqKBox& kb = H.ktab.box[b];
-            const int RX = 32 + kb.wxr - 1, RY = 4 * nw + kb.wyr - 1;
+            const int rx = iq_scan_rx(kb.wxr), ry = iq_scan_ry(kb.wyr, nw);
             for (int k = 2 * kb.s0; k < 2 * kb.s1; k++) {
               const IqChunk& c = chunks[k];
-              // x-runs: block layout x + RX (y + RY z); y-runs: y + RY (x + RX z)
-              kofs[k] = c.dir ? (((c.jz - kb.z0) * RX + (c.jx - kb.x0)) * RY + (c.jy - kb.y0)) | (1 << 30)
-                              : ((c.jz - kb.z0) * RY + (c.jy - kb.y0)) * RX + (c.jx - kb.x0);
+              kofs[k] = (c.jy - kb.y0) + ry * ((c.jx - kb.x0) + rx * (c.jz - kb.z0));
             }
           }
           pl->kofs_nw[nw] = pl->mem.upload(kofs.data(), kofs.size(), s);
@@ -1410,23 +1446,17 @@ void run_batch(iq_plan* pl, const IqQuery* hq, const IqQuery* q, int nq, bool ha
         }
         const int nw = pl->mfma_nw_forced ? pl->mfma_nw : pl->nw_tiles[ntile > 1 ? 2 : 1];
         const int YB = 4 * nw;
-        dim3 grid(nblk(g.dist[0], 32), nblk(g.dist[1], YB), (unsigned)(g.dist[2] * ntile));
+        const dim3 grid = scan_grid(pl, nf, nw);
         if (pl->prof) {
           HC(hipEventRecord(pl->prof_ev[pl->prof_used], s));
           // four 32-candidate row blocks per wavefront with a row inside the
           // grid, per x block and z x query tile: k-steps x (3 or 1) MFMAs
           double rows = 0.0;
           for (int y0 = 0; y0 < g.dist[1]; y0 += YB) rows += 4.0 * ((std::min(YB, g.dist[1] - y0) + 3) / 4);
-          pl->prof_mflop += (double)grid.x * rows * grid.z * pl->hd.ktab.nstep * (pl->mfma_split ? 3.0 : 1.0) *
+          pl->prof_mflop += (double)grid.x * rows * g.dist[2] * ntile * pl->hd.ktab.nstep * (pl->mfma_split ? 3.0 : 1.0) *
                             (2.0 * 32 * 32 * 16);
         }
-        if (pl->mfma_split)
-          hipLaunchKernelGGL((k_scan_mfma<true>), grid, dim3(64 * nw), pl->lds_nw[nw], s, D, q, nf, pl->mfma_gerr,
-                             pl->kofs_nw[nw]);
-        else
-          hipLaunchKernelGGL((k_scan_mfma<false>), grid, dim3(64 * nw), pl->lds_nw[nw], s, D, q, nf, pl->mfma_gerr,
-                             pl->kofs_nw[nw]);
-        HCL();
+        launch_scan_mfma(pl, q, nf, nw, s);
       } else {
         if (pl->prof) HC(hipEventRecord(pl->prof_ev[pl->prof_used], s));
         launch_scan_batch(pl, q, nf, s);
@@ -2233,13 +2263,7 @@ void harvest_queries(iq_plan* pl, std::vector<std::pair<int32_t, int32_t>> pool,
       const int ntile = (nq + 31) / 32;
       hipLaunchKernelGGL(k_mfma_bprep, dim3(pl->hd.ktab.nstep, ntile), dim3(64), 0, s, D, (const IqQuery*)dq, nq);
       const int nw = pl->mfma_nw_forced ? pl->mfma_nw : pl->nw_tiles[ntile > 1 ? 2 : 1];
-      dim3 grid(nblk(g.dist[0], 32), nblk(g.dist[1], 4 * nw), (unsigned)(g.dist[2] * ntile));
-      if (pl->mfma_split)
-        hipLaunchKernelGGL((k_scan_mfma<true>), grid, dim3(64 * nw), pl->lds_nw[nw], s, D, (const IqQuery*)dq, nq,
-                           pl->mfma_gerr, pl->kofs_nw[nw]);
-      else
-        hipLaunchKernelGGL((k_scan_mfma<false>), grid, dim3(64 * nw), pl->lds_nw[nw], s, D, (const IqQuery*)dq, nq,
-                           pl->mfma_gerr, pl->kofs_nw[nw]);
+      launch_scan_mfma(pl, dq, nq, nw, s);
     } else {
       launch_scan_batch(pl, dq, nq, s);
     }

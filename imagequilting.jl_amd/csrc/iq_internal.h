@@ -94,20 +94,28 @@ struct IqMapTile {
 };
 
 // MFMA scan: the K dimension is a list of 8-voxel chunks over the union of
-// all overlap masks, grouped by box; a chunk runs along x (dir 0) or y (dir 1).
+// all overlap masks, grouped by box; the chunks of a box are cy voxels along y
+// by 8 / cy along x (element e: y = e % cy, x = e / cy).
 struct IqChunk {
   int16_t jx, jy, jz;  // first voxel (tile coordinates)
-  int8_t dir, n;       // direction, valid voxels (0..8)
+  int8_t cy, ny, nx;   // shape, voxels inside the box along y and x (0: none)
 };
 struct IqKBox {
-  int32_t x0, y0, z0, wxr, wyr, wz;  // staged region of the box (x/y extents padded to the chunk runs)
+  int32_t x0, y0, z0, wxr, wyr, wz;  // the box (x/y extents padded to whole chunks)
   int32_t s0, s1;                    // k-steps [s0, s1) (two chunks per k-step)
+  int32_t cy;
 };
-#define IQ_MAX_KBOX 8
+#define IQ_MAX_KBOX 16
 struct IqKTab {
   int32_t nbox, nstep;
   IqKBox box[IQ_MAX_KBOX];
 };
+// The region of a box a group of nw wavefronts stages: rows of ry words along
+// y (an odd multiple of two, so that 8-byte reads of neighbouring rows fall on
+// different banks), one row per x.  The rows hold what the last wavefront's
+// last fragment read takes: wyr + 4 nw - 1 voxels.
+__host__ __device__ inline int iq_scan_ry(int wyr, int nw) { return (((wyr + 4 * nw) >> 1) | 1) << 1; }
+__host__ __device__ inline int iq_scan_rx(int wxr) { return 31 + wxr; }
 
 // Learned proposal: per overlap-mask shape a linear encoder e(x) = W x of
 // the masked values (IQ_EMB outputs) and the bank of encoded candidate
@@ -220,6 +228,7 @@ struct IqDev {
   // MFMA scan
   IqKTab ktab;
   const IqChunk* chunks;
+  const uint32_t* tiw;                     // the image as the scan stages it (k_scan_pack), y fastest
   const uint8_t* maskbits;                 // per mask: tilevox membership bytes
   uint4* bh;                               // B fragments (hi), [ntile][nstep][64]
   uint4* bl;                               // B fragments (lo)

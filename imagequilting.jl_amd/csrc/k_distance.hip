@@ -460,9 +460,17 @@ template __global__ void k_scan2_f32<4, 4, 16, 4>(const IqDev*, const IqQuery*, 
 // (hi*hi, hi*lo, lo*hi); bf16-exact data (small integer codes) needs one.
 // Each wavefront owns four 32-candidate rows (consecutive y) of one z, the
 // group (two to four wavefronts, chosen per plan so that the groups of a
-// launch pack the compute units evenly) 8 to 16 rows; the training-image block of each box
-// is staged in LDS as words (hi | lo << 16), and A fragments are gathered
-// from it along the chunk runs, so any run alignment works.
+// launch pack the compute units evenly) 8 to 16 rows; the block of each box is
+// staged in LDS from a packed copy of the image, y fastest, and A fragments
+// are read from it column by column (scan_frags).
+// What bounds it: split data the matrix cores at the card's power (70 % of the
+// cycles at 1.7 GHz for 2.9M candidates, 1.2 PFLOP/s issued, the rate of a large
+// library product), so LDS and permute work saved buys clock; bf16-exact data
+// the instructions around its four MFMAs a k-step.  Per launch, a region in the
+// image's order with eight words a row read, and this form: 2.9M candidates 65
+// queries 6,185 and 5,844 us; 302k candidates 26 queries 108 and 98 us; 403k
+// candidates, facies, 604 and 502 us.  Tried: two query tiles a group (bf16,
+// 180 registers: 21 % slower), four wavefronts per SIMD (equal).
 // Grid: x blocks (32), y blocks (4 x wavefronts), z = candidate z + dist_z * query tile.
 // ---------------------------------------------------------------------------
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 iq_bf16x8;
@@ -495,17 +503,18 @@ __device__ __forceinline__ void mfma_bprep_body(const IqDev* __restrict__ D, con
       const IqChunk ch = D->chunks[2 * step + (lane >> 5)];
       const uint8_t* mb = D->maskbits + (int64_t)st.mask * g.tilevox;
       const IqReal& R = D->reals[q.real];
-      if (ch.n > 0) {
+      if (ch.nx > 0) {
         // mask bytes, then grid values of the chunk's (up to) eight voxels,
-        // each batch of loads in flight together; positions past the chunk
-        // repeat its last voxel and are dropped
+        // each batch of loads in flight together; positions past the box
+        // repeat its first voxel and are dropped
         int64_t gi[8];
         uint8_t on[8];
 #pragma unroll
         for (int e = 0; e < 8; e++) {
-          const int ee = e < ch.n ? e : ch.n - 1;
-          const int x = ch.jx + (ch.dir == 0 ? ee : 0), y = ch.jy + (ch.dir == 1 ? ee : 0), z = ch.jz;
-          on[e] = mb[x + g.tile[0] * (y + g.tile[1] * z)];
+          const int ey = e & (ch.cy - 1), ex = e / ch.cy;
+          const bool in = ey < ch.ny && ex < ch.nx;
+          const int x = ch.jx + (in ? ex : 0), y = ch.jy + (in ? ey : 0), z = ch.jz;
+          on[e] = in ? mb[x + g.tile[0] * (y + g.tile[1] * z)] : 0;
           gi[e] = iq_lin3(R.pad, st.origin[0] + x, st.origin[1] + y, st.origin[2] + z);
         }
         float v[8];
@@ -520,7 +529,7 @@ __device__ __forceinline__ void mfma_bprep_body(const IqDev* __restrict__ D, con
         }
 #pragma unroll
         for (int e = 0; e < 8; e++) {
-          if (e >= ch.n || !on[e]) continue;
+          if (!on[e]) continue;
           const uint32_t wv = iq_split_word(v[e]);
           h[e >> 1] |= (wv & 0xffffu) << (16 * (e & 1));
           l[e >> 1] |= (wv >> 16) << (16 * (e & 1));
@@ -566,14 +575,67 @@ k_a2_f32(const double* __restrict__ a2, const uint8_t* __restrict__ disabled, in
     out[c] = disabled[c] ? __builtin_nanf("") : (float)a2[c];
 }
 
+// The image in the words the scan stages, y fastest: word (y, x, z) holds the
+// bf16 split (hi | lo << 16) of its voxel (SPLIT), or its voxel and the next
+// along y as a bf16 pair (bf16-exact data).  Written once per plan; `n` words,
+// those past the image zero (a staged region may run past it).
+template <bool SPLIT>
+__global__ void __launch_bounds__(256)
+k_scan_pack(const float* __restrict__ ti, int t0, int t1, int t2, uint32_t* __restrict__ out, int64_t n) {
+  const int64_t nv = (int64_t)t0 * t1 * t2;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+    uint32_t v = 0;
+    if (i < nv) {
+      const int y = (int)(i % t1), x = (int)((i / t1) % t0), z = (int)(i / ((int64_t)t0 * t1));
+      const float* p = ti + x + (int64_t)t0 * (y + (int64_t)t1 * z);
+      if (SPLIT) v = iq_split_word(*p);
+      else v = iq_bf16_rne(*p) | (y + 1 < t1 ? iq_bf16_rne(p[t0]) << 16 : 0u);
+    }
+    out[i] = v;
+  }
+}
+template __global__ void k_scan_pack<true>(const float*, int, int, int, uint32_t*, int64_t);
+template __global__ void k_scan_pack<false>(const float*, int, int, int, uint32_t*, int64_t);
+
+// A fragments of four candidate rows (consecutive y) for one chunk, taken as
+// four pairs of voxels along y, off[c] words from the lane's first: whatever
+// the chunk's shape the code is the same, without a branch between the reads
+// and the MFMAs (one by shape cost a fifth of the kernel's time).  The rows'
+// pairs overlap, so a pair takes five words for the four rows together, 20 a
+// chunk; a chunk along x takes 8 words a row, 32.  at and off are even: 8-byte
+// reads.
+typedef unsigned int iq_u32x2 __attribute__((ext_vector_type(2)));
+template <bool SPLIT>
+__device__ __forceinline__ void scan_frags(const uint32_t* lw, int at, const int (&off)[4], uint4 (&h)[4], uint4 (&l)[4]) {
+  uint32_t w[4][6];
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    const uint32_t* p = lw + at + off[c];
+    const iq_u32x2 v0 = ((const iq_u32x2*)p)[0], v1 = ((const iq_u32x2*)p)[1];
+    w[c][0] = v0.x; w[c][1] = v0.y; w[c][2] = v1.x; w[c][3] = v1.y;
+    if (SPLIT) w[c][4] = p[4];
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    uint32_t a[4], b[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      a[c] = SPLIT ? __builtin_amdgcn_perm(w[c][i + 1], w[c][i], 0x05040100u) : w[c][i];
+      b[c] = SPLIT ? __builtin_amdgcn_perm(w[c][i + 1], w[c][i], 0x07060302u) : 0u;
+    }
+    h[i] = make_uint4(a[0], a[1], a[2], a[3]);
+    if (SPLIT) l[i] = make_uint4(b[0], b[1], b[2], b[3]);
+  }
+}
+
 template <bool SPLIT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 k_scan_mfma(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int nq, double gerr,
             const int32_t* __restrict__ kofs_tab) {
-  extern __shared__ uint32_t lw[];
+  extern __shared__ __align__(16) uint32_t lw[];
   __shared__ float red[4][32];
   const IqGeo& g = D->g;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int row = lane & 31, kb = lane >> 5;
   const int tile = blockIdx.z / g.dist[2];
   const int cz = blockIdx.z % g.dist[2];
@@ -581,10 +643,12 @@ k_scan_mfma(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int nq,
   const int cx0 = blockIdx.x * 32, cy0 = blockIdx.y * 4 * nw;
   const bool wlive = cy0 + 4 * w < g.dist[1];  // uniform per wavefront
   const int nstep = D->ktab.nstep;
-  const int t0 = g.ti[0], t1 = g.ti[1], t2 = g.ti[2];
+  const int t0 = g.ti[0], t1 = g.ti[1];
   const int d0 = g.dist[0], d1 = g.dist[1];
-  const auto ti = iq_glob(D->ti32);
-  constexpr int SU = 8;
+  const auto tiw = iq_glob(D->tiw);
+  const auto kofs = iq_glob(kofs_tab);
+  const auto bhp = iq_glob((const iq_u32x4*)(D->bh + (int64_t)tile * nstep * 64 + lane));
+  const auto blp = iq_glob((const iq_u32x4*)(D->bl + (int64_t)tile * nstep * 64 + lane));
   iq_f32x16 acc[4];
 #pragma unroll
   for (int i = 0; i < 4; i++)
@@ -592,101 +656,84 @@ k_scan_mfma(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int nq,
     for (int v = 0; v < 16; v++) acc[i][v] = 0.0f;
   for (int b = 0; b < D->ktab.nbox; b++) {
     const IqKBox kbx = D->ktab.box[b];
-    const int RX = 32 + kbx.wxr - 1, RY = 4 * nw + kbx.wyr - 1;
-    const int n = RX * RY * kbx.wz;
-    const int gx0 = cx0 + kbx.x0, gy0 = cy0 + kbx.y0, gz0 = cz + kbx.z0;
-    // A box's chunks all run along x or all along y.  The block is staged so
-    // that a run is contiguous: x-runs in the layout x + RX (y + RY z),
-    // y-runs in y + RY (x + RX z); a wavefront's four rows then sit at a
-    // uniform stride (RX, or 1) and the eight words of a run at immediate
-    // offsets.  Element i = x + RX (y + RY z) of the walk; coordinates
-    // advance incrementally (NT per element, SU elements per pass with all
-    // their loads issued first); windows past the training image read as zero.
-    const auto kofs = iq_glob(kofs_tab);
-    const bool ydir = kbx.s0 < kbx.s1 && (kofs[2 * kbx.s0] >> 30) != 0;
-    int x = (int)threadIdx.x % RX, y = ((int)threadIdx.x / RX) % RY, z = (int)threadIdx.x / (RX * RY);
-    const int sx = NT % RX, sy = (NT / RX) % RY, sz = NT / (RX * RY);
-    for (int i0 = threadIdx.x; i0 < n; i0 += NT * SU) {
-      float v[SU];
-      bool in[SU];
-      int at[SU];
-#pragma unroll
-      for (int u = 0; u < SU; u++) {
-        const int gx = gx0 + x, gy = gy0 + y, gz = gz0 + z;
-        in[u] = gx < t0 && gy < t1 && gz < t2;
-        v[u] = ti[in[u] ? gx + (int64_t)t0 * (gy + (int64_t)t1 * gz) : 0];
-        at[u] = ydir ? y + RY * (x + RX * z) : i0 + NT * u;
-        x += sx;
+    const int ry = iq_scan_ry(kbx.wyr, nw), rx = iq_scan_rx(kbx.wxr);
+    // The box's region goes straight to LDS, a word a lane, all loads in
+    // flight (no registers, no tests: the packed image has room past its end,
+    // and what a candidate outside the grid reads does not matter).
+    {
+      const int n = ry * rx * kbx.wz;
+      int y = (int)threadIdx.x % ry, x = (int)threadIdx.x / ry % rx, z = (int)threadIdx.x / (ry * rx);
+      const int sy = NT % ry, sx = NT / ry % rx, sz = NT / (ry * rx);
+      int gi = cy0 + kbx.y0 + y + t1 * (cx0 + kbx.x0 + x + t0 * (cz + kbx.z0 + z));
+      const int sg = sy + t1 * (sx + t0 * sz);
+      if (b) __syncthreads();  // the previous box's region is no longer read
+      for (int i0 = 64 * w; i0 < n; i0 += NT) {
+        if (i0 + lane < n)
+          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(tiw + gi),
+                                           (__attribute__((address_space(3))) void*)(lw + i0), 4, 0, 0);
         y += sy;
-        z += sz;
-        if (x >= RX) { x -= RX; y++; }
-        if (y >= RY) { y -= RY; z++; }
+        x += sx;
+        gi += sg;
+        if (y >= ry) { y -= ry; x++; gi += t1 - ry; }
+        if (x >= rx) { x -= rx; gi += t1 * (t0 - rx); }
       }
-#pragma unroll
-      for (int u = 0; u < SU; u++)
-        if (i0 + NT * u < n) lw[at[u]] = iq_split_word(in[u] ? v[u] : 0.0f);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
     }
-    __syncthreads();
-    // B fragments and chunk offsets are loaded one k-step ahead
-    const auto bhp = iq_glob((const iq_u32x4*)(D->bh + (int64_t)tile * nstep * 64 + lane));
-    const auto blp = iq_glob((const iq_u32x4*)(D->bl + (int64_t)tile * nstep * 64 + lane));
-    const int lane_off = ydir ? 4 * w + RY * row : 4 * w * RX + row;
-    const int istr = ydir ? 1 : RX;
-    iq_u32x4 bh_n = {0u, 0u, 0u, 0u}, bl_n = {0u, 0u, 0u, 0u};
-    int ko_n = 0;
-    if (kbx.s0 < kbx.s1) {
-      bh_n = bhp[(int64_t)kbx.s0 * 64];
-      if (SPLIT) bl_n = blp[(int64_t)kbx.s0 * 64];
-      ko_n = kofs[2 * kbx.s0 + kb];
-    }
-    for (int step = kbx.s0; step < kbx.s1; step++) {
-      const iq_bf16x8 bh = __builtin_bit_cast(iq_bf16x8, bh_n);
-      iq_bf16x8 bl;
-      if (SPLIT) bl = __builtin_bit_cast(iq_bf16x8, bl_n);
-      const int ko = ko_n;
-      if (step + 1 < kbx.s1) {
-        bh_n = bhp[(int64_t)(step + 1) * 64];
-        if (SPLIT) bl_n = blp[(int64_t)(step + 1) * 64];
-        ko_n = kofs[2 * (step + 1) + kb];
-      }
-      const int base = (ko & 0x3fffffff) + lane_off;
-      if (!wlive) continue;  // every candidate row of this wavefront is past the grid
-      // all 32 LDS words of the four row blocks first, then the MFMAs in an
-      // order where consecutive ones use different accumulators
-      uint32_t wv[4][8];
+    if (!wlive) continue;  // every candidate row of this wavefront is past the grid
+    const int lane_off = 4 * w + ry * row;
+    int off[4];  // the chunk's pairs of voxels: cy / 2 a column
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int rb = base + i * istr;
+    for (int c = 0; c < 4; c++) off[c] = 2 * c % kbx.cy + ry * (2 * c / kbx.cy);
+    // k-steps: B fragments and chunk offsets are loaded ahead, one step for
+    // split data (a step's twelve MFMAs cover the load: two ahead measured 8 %
+    // slower), two for the four MFMAs of bf16-exact data (6 % faster);
+    // consecutive MFMAs use different accumulators
+    iq_u32x4 bh[2], bl[2];
+    int ko[2];
+    auto fetch = [&](int u, int step) {
+      bh[u] = bhp[(int64_t)step * 64];
+      if (SPLIT) bl[u] = blp[(int64_t)step * 64];
+      ko[u] = kofs[2 * step + kb];
+    };
+    auto mfmas = [&](int u) {
+      uint4 h[4], l[4];
+      scan_frags<SPLIT>(lw, ko[u] + lane_off, off, h, l);
+      const iq_bf16x8 qh = __builtin_bit_cast(iq_bf16x8, bh[u]);
 #pragma unroll
-        for (int e = 0; e < 8; e++) wv[i][e] = lw[rb + e];
-      }
-      iq_bf16x8 ah[4], al[4];
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        uint4 h4, l4;
-        h4.x = __builtin_amdgcn_perm(wv[i][1], wv[i][0], 0x05040100u);
-        h4.y = __builtin_amdgcn_perm(wv[i][3], wv[i][2], 0x05040100u);
-        h4.z = __builtin_amdgcn_perm(wv[i][5], wv[i][4], 0x05040100u);
-        h4.w = __builtin_amdgcn_perm(wv[i][7], wv[i][6], 0x05040100u);
-        ah[i] = __builtin_bit_cast(iq_bf16x8, h4);
-        if (SPLIT) {
-          l4.x = __builtin_amdgcn_perm(wv[i][1], wv[i][0], 0x07060302u);
-          l4.y = __builtin_amdgcn_perm(wv[i][3], wv[i][2], 0x07060302u);
-          l4.z = __builtin_amdgcn_perm(wv[i][5], wv[i][4], 0x07060302u);
-          l4.w = __builtin_amdgcn_perm(wv[i][7], wv[i][6], 0x07060302u);
-          al[i] = __builtin_bit_cast(iq_bf16x8, l4);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < 4; i++) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bh, acc[i], 0, 0, 0);
+      for (int i = 0; i < 4; i++)
+        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(iq_bf16x8, h[i]), qh, acc[i], 0, 0, 0);
       if (SPLIT) {
+        const iq_bf16x8 ql = __builtin_bit_cast(iq_bf16x8, bl[u]);
 #pragma unroll
-        for (int i = 0; i < 4; i++) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bl, acc[i], 0, 0, 0);
+        for (int i = 0; i < 4; i++)
+          acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(iq_bf16x8, h[i]), ql, acc[i], 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < 4; i++) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[i], bh, acc[i], 0, 0, 0);
+        for (int i = 0; i < 4; i++)
+          acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(iq_bf16x8, l[i]), qh, acc[i], 0, 0, 0);
       }
+    };
+    const int s0 = kbx.s0, s1 = kbx.s1;
+    if (s0 < s1) fetch(SPLIT ? 1 : 0, s0);
+    if (!SPLIT && s0 + 1 < s1) fetch(1, s0 + 1);
+    if constexpr (SPLIT) {
+      for (int step = s0; step < s1; step++) {
+        bh[0] = bh[1];
+        bl[0] = bl[1];
+        ko[0] = ko[1];
+        if (step + 1 < s1) fetch(1, step + 1);
+        mfmas(0);
+      }
+    } else {
+      int step = s0;
+      for (; step + 1 < s1; step += 2) {
+        mfmas(0);
+        if (step + 2 < s1) fetch(0, step + 2);
+        mfmas(1);
+        if (step + 3 < s1) fetch(1, step + 3);
+      }
+      if (step < s1) mfmas(0);
     }
-    __syncthreads();
   }
   // epilogue: lane holds C[row'][col] for col = lane % 32 (its query)
   const int qi = tile * 32 + row;
