@@ -345,6 +345,18 @@ bool fits_range(const float* v, int64_t n) {
   return true;
 }
 
+// Integer codes small enough that every sum and difference of the distance
+// over V voxels is an integer below 2^24: the scan's FP32 distances are then
+// the exact ones, in whatever order they are summed.
+bool exact_codes(const float* v, int64_t n, int V) {
+  float m = 0.0f;
+  for (int64_t i = 0; i < n; i++) {
+    if (v[i] != std::floor(v[i])) return false;
+    m = std::max(m, std::fabs(v[i]));
+  }
+  return 4.0 * (double)V * (double)m * (double)m < 0x1p24;
+}
+
 // Relative error bound of the MFMA scan's correlation: |AB32 - AB| <=
 // scan_gerr * sum |a||b| over a mask of nstep k-steps (16 voxels each).
 //  * Accumulation: every bf16 x bf16 product is exact in FP32; the FP32 sums
@@ -406,6 +418,7 @@ struct iq_plan {
   double tol = 0.1;
   int naux = 0;
   bool fast = false;
+  bool exact_int = false;  // the MFMA scan's FP32 distances are exact (integer codes)
   bool rounded = false;  // fast, on the FP32 rounding of Float64 data (MFMA scan only)
   bool hard = false;
   bool any_multi = false;
@@ -540,7 +553,7 @@ dim3 scan_grid(const iq_plan* pl, int nq, int nw) {
 void launch_scan_mfma(iq_plan* pl, const IqQuery* q, int nq, int nw, hipStream_t s) {
   hipLaunchKernelGGL((pl->mfma_split ? k_scan_mfma<true> : k_scan_mfma<false>),
                      scan_grid(pl, nq, nw), dim3(64 * nw), pl->lds_nw[nw], s, (const IqDev*)pl->dd, q, nq, pl->mfma_gerr,
-                     pl->kofs_nw[nw]);
+                     pl->kofs_nw[nw], pl->exact_int ? 1 : 0);
   HCL();
 }
 
@@ -923,6 +936,8 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
   H.g = g;
   const double* tid = (const double*)d->ti;
   const float* tif = (const float*)d->ti;
+  int vmax = 0;  // voxels of the largest overlap mask
+  for (const HostMask& hm : hmasks) vmax = std::max(vmax, hm.V);
   bool exact16 = false;  // fast, and every value a bf16 (decided on the host's copy: reading the device's costs 1 us a value)
   if (d->ti_dtype == IQ_F32) {
     H.ti = pl->mem.upload(tif, tivox, s);
@@ -930,6 +945,7 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
     if (pl->fast) {
       H.ti32 = (const float*)H.ti;
       exact16 = bf16_exact(tif, tivox);
+      pl->exact_int = exact16 && exact_codes(tif, tivox, vmax);
     }
   } else {
     H.ti = pl->mem.upload(tid, tivox, s);
@@ -939,6 +955,7 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
       std::vector<float> t32((size_t)tivox);
       for (int64_t i = 0; i < tivox; i++) t32[i] = (float)tid[i];
       exact16 = bf16_exact(t32.data(), tivox);
+      pl->exact_int = exact16 && !pl->rounded && exact_codes(t32.data(), tivox, vmax);
       H.ti32 = pl->mem.upload(t32.data(), tivox, s);
       HC(hipStreamSynchronize(s));
     }
@@ -1472,10 +1489,10 @@ void run_batch(iq_plan* pl, const IqQuery* hq, const IqQuery* q, int nq, bool ha
         pl->batch_flop.push_back(f);
         pl->prof_flop += f;
       }
-      hipLaunchKernelGGL(k_band_select, dim3(nblk(P, 256 * SEL_PT), nf), dim3(256), 0, s, D, q);
+      const bool exact = pl->mfma && pl->exact_int;
+      hipLaunchKernelGGL(k_band_select, dim3(nblk(P, 256 * SEL_PT), nf), dim3(256), 0, s, D, q, exact ? 1 : 0);
       HCL();
-      launch_recheck(pl, q, nf, s);
-      HCL();
+      if (!exact) launch_recheck(pl, q, nf, s);
     } else {
       hipLaunchKernelGGL(k_band_all, dim3(nblk(P, 256), nf), dim3(256), 0, s, D, q);
       HCL();

@@ -631,7 +631,7 @@ __device__ __forceinline__ void scan_frags(const uint32_t* lw, int at, const int
 template <bool SPLIT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 k_scan_mfma(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int nq, double gerr,
-            const int32_t* __restrict__ kofs_tab) {
+            const int32_t* __restrict__ kofs_tab, int exact) {
   extern __shared__ __align__(16) uint32_t lw[];
   __shared__ float red[4][32];
   const IqGeo& g = D->g;
@@ -780,6 +780,19 @@ k_scan_mfma(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int nq,
           const int ox = 8 * (v >> 2) + (v & 3);
           A[v] = a2f[ox < xl ? rb + ox : rb - 4 * kb];
         }
+        if (exact) {  // uniform: every operand and result is an integer below 2^24
+#pragma unroll
+          for (int v = 0; v < 16; v++) {
+            const int ox = 8 * (v >> 2) + (v & 3);
+            float d = __builtin_fabsf(__builtin_fmaf(-2.0f, acc[i][v], A[v]) + B);
+            if (A[v] != A[v]) d = __builtin_inff();
+            if (ox < xl) {
+              lo_out[rb + ox] = d;
+              lmin = fminf(lmin, d);
+            }
+          }
+          continue;
+        }
 #pragma unroll
         for (int v = 0; v < 16; v++) {
           const int ox = 8 * (v >> 2) + (v & 3);
@@ -808,8 +821,8 @@ k_scan_mfma(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int nq,
   }
 }
 
-template __global__ void k_scan_mfma<true>(const IqDev*, const IqQuery*, int, double, const int32_t*);
-template __global__ void k_scan_mfma<false>(const IqDev*, const IqQuery*, int, double, const int32_t*);
+template __global__ void k_scan_mfma<true>(const IqDev*, const IqQuery*, int, double, const int32_t*, int);
+template __global__ void k_scan_mfma<false>(const IqDev*, const IqQuery*, int, double, const int32_t*, int);
 
 #define IQ_SCAN_INST(R, LX, LY, LZ) \
   template __global__ void k_scan_f32<R, LX, LY, LZ>(const IqDev*, const IqQuery*, int);
@@ -822,11 +835,14 @@ IQ_SCAN_INST(4, 8, 16, 2)
 // Band superset: lo <= T where T = round_up(fl(fl(1+tol) * U)) and U is the
 // least upper bound of the scan, so every exact band member is selected.
 // One bitmap bit per candidate (ballot words of 64 candidates) and an
-// unordered list of the members.  Grid: (candidate blocks, query).
+// unordered list of the members, one reservation a wavefront.  `exact`: the
+// scan's values are the exact distances (integer codes), so members get theirs
+// here, with the exact minimum, and no recheck follows.
+// Grid: (candidate blocks, query).
 // ---------------------------------------------------------------------------
 #define SEL_PT 8
 __global__ void __launch_bounds__(256)
-k_band_select(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
+k_band_select(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int exact) {
   const IqQuery q = qs[blockIdx.y];
   const IqStep& st = D->steps[q.step];
   if (q.multi || st.mask < 0) return;
@@ -836,6 +852,8 @@ k_band_select(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
   const float Tf = iq_f32_up((1.0 + D->tol) * U);
   const auto lo = iq_glob(D->lo32 + slot * P);
   const int lane = threadIdx.x & 63;
+  if (exact && blockIdx.x == 0 && threadIdx.x == 0)
+    D->gmin64[slot] = (unsigned long long)__double_as_longlong(U);
   // a wavefront covers SEL_PT words of 64 consecutive candidates
   const int64_t c0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 64 * SEL_PT + lane;
   float v[SEL_PT];
@@ -844,18 +862,27 @@ k_band_select(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
     const int64_t c = c0 + 64 * j;
     v[j] = lo[c < P ? c : 0];
   }
+  unsigned long long bal[SEL_PT];
+  int total = 0;
 #pragma unroll
   for (int j = 0; j < SEL_PT; j++) {
     const int64_t c = c0 + 64 * j;
-    const bool sel = c < P && v[j] <= Tf;
-    const unsigned long long bal = __ballot(sel);
-    if (lane == 0 && (c >> 6) < D->nw64) D->bitmap[slot * D->nw64 + (c >> 6)] = bal;
-    if (bal) {
-      int base = 0;
-      if (lane == 0) base = atomicAdd(&D->nsup[slot], __popcll(bal));
-      base = __shfl(base, 0);
-      if (sel) D->sup[slot * P + base + __popcll(bal & ((1ull << lane) - 1ull))] = (int32_t)c;
+    bal[j] = __ballot(c < P && v[j] <= Tf);
+    total += __popcll(bal[j]);
+    if (lane == 0 && (c >> 6) < D->nw64) D->bitmap[slot * D->nw64 + (c >> 6)] = bal[j];
+  }
+  if (!total) return;  // uniform
+  int base = 0;
+  if (lane == 0) base = atomicAdd(&D->nsup[slot], total);
+  base = __builtin_amdgcn_readfirstlane(base);
+#pragma unroll
+  for (int j = 0; j < SEL_PT; j++) {
+    const int64_t c = c0 + 64 * j;
+    if ((bal[j] >> lane) & 1ull) {
+      D->sup[slot * P + base + __popcll(bal[j] & ((1ull << lane) - 1ull))] = (int32_t)c;
+      if (exact) D->dexact[slot * P + c] = (double)v[j];
     }
+    base += __popcll(bal[j]);
   }
 }
 
