@@ -2963,7 +2963,9 @@ int iq_relaxation(iq_ctx* ctx, const double* D, const double* const* Ds, int nau
     int64_t* cnt = m.alloc<int64_t>(1);
     int32_t* err = m.alloc<int32_t>(1);
     HC(hipMemsetAsync(err, 0, sizeof(int32_t), s));
-    hipLaunchKernelGGL(k_relax_host, dim3(1), dim3(FB), 0, s, n, nsrc, dmaps, tol, bits, ev, cnt, err);
+    uint64_t* lkey = m.alloc<uint64_t>(n);
+    int32_t* lidx = m.alloc<int32_t>(n);
+    hipLaunchKernelGGL(k_relax_host, dim3(1), dim3(FB), 0, s, n, nsrc, dmaps, tol, bits, ev, lkey, lidx, cnt, err);
     HCL();
     int32_t code = 0;
     int64_t c = 0;

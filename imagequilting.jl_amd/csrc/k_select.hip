@@ -579,12 +579,18 @@ k_band_finalize(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int
 // then index: Julia's Perm ordering for partialsortperm, relaxation.jl:12,27),
 // and a prefix of length m is { i : (bits(v_i), i) <= the m-th smallest
 // pair }: non-negative doubles and +inf order like their IEEE bit patterns.
-// So each set needs one order statistic (radix selection, blk_kth_key) and
-// one pass that writes it as a bitmap (bits: nsrc maps of nwd words); the
+// So each set needs one order statistic (bracketed by a sample, or by radix
+// selection, blk_kth_key) and one pass that writes it as a bitmap (bits: nsrc maps of nwd words); the
 // running intersection is the AND of the bitmaps.
 // ---------------------------------------------------------------------------
 #define KS_CAP 512          // bins this small are ranked pairwise in LDS
-#define KS_LDS_WORDS 1792   // 64-bit LDS words: histogram 2048 x u32, KS_CAP values, KS_CAP indices
+#define KS_SAMPLE 4096      // sample of a map from which its order statistic is bracketed
+// Smaller maps are selected without a sample: two sources take 66 us without
+// and 79 us with it at 16,384 values, 112 and 107 at 32,768, 150 and 105 at
+// 65,536, 544 and 289 at 262,144.
+#define KS_MIN 32768
+#define KS_U 8              // loads in flight per work-item in the passes over a map
+#define KS_LDS_WORDS 3072   // 64-bit LDS words: histogram 2048 x u32, then the sample (u32), or KS_CAP values and indices
 
 __device__ inline uint64_t f64_bits(double x) { return (uint64_t)__double_as_longlong(x); }
 
@@ -636,12 +642,12 @@ __device__ __forceinline__ void blk_kth_key(const double* __restrict__ map, int6
     const uint32_t dm = (1u << w) - 1u;
     for (int b = threadIdx.x; b < (1 << w); b += FB) hist[b] = 0u;
     __syncthreads();
-    for (int64_t i0 = threadIdx.x; i0 < P; i0 += 8 * FB) {
-      uint64_t v[8];
+    for (int64_t i0 = threadIdx.x; i0 < P; i0 += KS_U * FB) {
+      uint64_t v[KS_U];
 #pragma unroll
-      for (int k = 0; k < 8; k++) v[k] = i0 + k * FB < P ? f64_bits(mg[i0 + k * FB]) : 0ull;
+      for (int k = 0; k < KS_U; k++) v[k] = i0 + k * FB < P ? f64_bits(mg[i0 + k * FB]) : 0ull;
 #pragma unroll
-      for (int k = 0; k < 8; k++) {
+      for (int k = 0; k < KS_U; k++) {
         const bool mt = i0 + k * FB < P && (v[k] & hm) == pv;
         const uint32_t d = (uint32_t)(v[k] >> sft) & dm;
         // lanes sharing the first matching lane's digit add once, through it
@@ -763,21 +769,172 @@ __device__ __forceinline__ void blk_prefix_bits(const double* __restrict__ map, 
   }
 }
 
+// The same prefix set written by one pass over the map.  A strided sample
+// brackets the m-th smallest value (3.2 standard deviations of its rank either
+// side, on the top 32 bits); the pass writes the bits of everything below the
+// bracket and lists what falls inside (lkey, lidx: room for P), and the order
+// statistic is found in the list, whose members then get their bits.  The
+// passes over the maps are what the relaxation costs, and the radix selection
+// takes four: 336 queries of 3 maps of 216,225 values took 988 us that way,
+// 684 us this way (the bits and the list are what a pass writes).  False, with
+// the bits to be written again, when the bracket missed or too many members tie.
+__device__ __forceinline__ bool blk_prefix_sampled(const double* __restrict__ map, int64_t P, int64_t m, uint32_t* __restrict__ bits,
+                                                   uint64_t* __restrict__ lkey, int32_t* __restrict__ lidx, uint64_t* lds,
+                                                   SelScratch& sh) {
+  if (P < KS_MIN) return false;
+  uint32_t* hist = (uint32_t*)lds;
+  uint32_t* smp = (uint32_t*)(lds + 1024);
+  const auto* mg = iq_glob(map);
+  const int lane = threadIdx.x & 63;
+  for (int i = threadIdx.x; i < KS_SAMPLE; i += FB) smp[i] = (uint32_t)(f64_bits(mg[(int64_t)i * P / KS_SAMPLE]) >> 32);
+  const double pr = (double)m / (double)P, mean = pr * KS_SAMPLE, dev = 3.2 * __builtin_sqrt(mean * (1.0 - pr)) + 2.0;
+  uint32_t br[2] = {0u, 0xffffffffu};
+  __syncthreads();
+  for (int side = 0; side < 2; side++) {
+    const double rk = side == 0 ? mean - dev : mean + dev;
+    if (rk < 1.0 || rk > (double)KS_SAMPLE) continue;  // open on this side
+    int64_t r = (int64_t)rk, cnt;
+    uint32_t pv = 0, hm = 0;
+    for (int known = 0; known < 32;) {  // digits of 11, 11 and 10 bits
+      const int w = 32 - known >= 11 ? 11 : 32 - known, sft = 32 - known - w;
+      for (int b = threadIdx.x; b < (1 << w); b += FB) hist[b] = 0u;
+      __syncthreads();
+      for (int i = threadIdx.x; i < KS_SAMPLE; i += FB)
+        if ((smp[i] & hm) == pv) atomicAdd(&hist[(smp[i] >> sft) & ((1u << w) - 1u)], 1u);
+      __syncthreads();
+      const int bin = blk_find_bin(hist, 1 << w, r, cnt, sh);
+      pv |= (uint32_t)bin << sft;
+      hm |= ((1u << w) - 1u) << sft;
+      known += w;
+    }
+    br[side] = pv;
+  }
+  const uint32_t lo = br[0], hi = br[1];
+  if (lo == hi) return false;  // tied values
+  if (threadIdx.x == 0) sh.flag = 0;
+  __syncthreads();
+  const int64_t nwd = (P + 31) / 32;
+  int64_t below = 0;
+  for (int64_t base0 = (int64_t)(threadIdx.x >> 6) * 64; base0 < P; base0 += KS_U * FB) {
+    uint64_t v[KS_U];
+#pragma unroll
+    for (int k = 0; k < KS_U; k++) {
+      const int64_t i = base0 + k * FB + lane;
+      v[k] = i < P ? f64_bits(mg[i]) : ~0ull;
+    }
+#pragma unroll
+    for (int k = 0; k < KS_U; k++) {
+      const int64_t base = base0 + k * FB, i = base + lane;
+      const uint32_t h = (uint32_t)(v[k] >> 32);
+      const uint64_t b = __ballot(i < P && h < lo);
+      if (lane == 0 && base < P) {
+        const int64_t w = base >> 5;
+        bits[w] = (uint32_t)b;
+        if (w + 1 < nwd) bits[w + 1] = (uint32_t)(b >> 32);
+        below += __popcll(b);
+      }
+      const bool in = i < P && h >= lo && h <= hi;
+      const uint64_t c = __ballot(in);
+      if (c) {
+        int at = 0;
+        if (lane == 0) at = atomicAdd(&sh.flag, __popcll(c));
+        at = __builtin_amdgcn_readfirstlane(at);
+        if (in) {
+          const int slot = at + __popcll(c & ((1ull << lane) - 1ull));
+          lkey[slot] = v[k];
+          lidx[slot] = (int32_t)i;
+        }
+      }
+    }
+  }
+  const int64_t nb = blk_sum_i64(below, sh);  // its barriers also publish the list
+  const int n = sh.flag;
+  __syncthreads();  // flag is reset below
+  int64_t r = m - nb, cnt = n;
+  if (r < 1 || r > n) { __syncthreads(); return false; }
+  // the r-th smallest (value, index) pair of the list
+  uint64_t* cv = lds + 1024;
+  uint32_t* ci = (uint32_t*)(lds + 1024 + KS_CAP);
+  int known = lo == hi ? 32 : __builtin_clz(lo ^ hi);  // leading bits the bracket fixes
+  uint64_t hm = known ? ~0ull << (64 - known) : 0ull, pv = ((uint64_t)lo << 32) & hm;
+  while (known < 64 && cnt > KS_CAP) {
+    const int w = 64 - known >= 11 ? 11 : 64 - known;
+    const int sft = 64 - known - w;
+    const uint32_t dm = (1u << w) - 1u;
+    for (int b = threadIdx.x; b < (1 << w); b += FB) hist[b] = 0u;
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += FB) {
+      const uint64_t v = lkey[i];
+      if ((v & hm) == pv) atomicAdd(&hist[(uint32_t)(v >> sft) & dm], 1u);
+    }
+    __syncthreads();
+    const int bin = blk_find_bin(hist, 1 << w, r, cnt, sh);
+    pv |= (uint64_t)bin << sft;
+    hm |= (uint64_t)dm << sft;
+    known += w;
+  }
+  if (cnt > KS_CAP) { __syncthreads(); return false; }
+  if (threadIdx.x == 0) sh.flag = 0;
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += FB) {
+    const uint64_t v = lkey[i];
+    if ((v & hm) == pv) {
+      const int slot = atomicAdd(&sh.flag, 1);
+      cv[slot] = v;
+      ci[slot] = (uint32_t)lidx[i];
+    }
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < (int)cnt) {
+    const uint64_t myv = cv[threadIdx.x];
+    const uint32_t myi = ci[threadIdx.x];
+    int rank = 0;
+    for (int f = 0; f < (int)cnt; f++) rank += (cv[f] < myv || (cv[f] == myv && ci[f] < myi)) ? 1 : 0;
+    if (rank == r - 1) { sh.result = myi; sh.aux = (int64_t)myv; }
+  }
+  __syncthreads();
+  const uint64_t tv = (uint64_t)sh.aux;
+  const int64_t ti = sh.result;
+  for (int i = threadIdx.x; i < n; i += FB) {
+    const uint64_t v = lkey[i];
+    const int32_t c = lidx[i];
+    if (v < tv || (v == tv && c <= ti)) atomicOr(&bits[c >> 5], 1u << (c & 31));
+  }
+  __syncthreads();
+  return true;
+}
+
+// One word of a prefix set's bits (past the vector cache: set by atomics).
+__device__ inline uint32_t ks_word(const uint32_t* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The prefix set of length m as bits.
+__device__ __forceinline__ void blk_prefix(const double* __restrict__ map, int64_t P, int64_t m, uint32_t* __restrict__ bits,
+                                           uint64_t* lkey, int32_t* lidx, uint64_t* lds, SelScratch& sh) {
+  if (m > 0 && blk_prefix_sampled(map, P, m, bits, lkey, lidx, lds, sh)) return;
+  uint64_t tv = 0;
+  int64_t ti = -1;  // empty prefix
+  if (m > 0) blk_kth_key(map, P, m, lds, sh, &tv, &ti);
+  blk_prefix_bits(map, P, tv, ti, bits);
+  __syncthreads();
+}
+
 // Returns the size of the database written to ev (ascending), -1 if every
-// candidate is disabled.  lds: KS_LDS_WORDS 64-bit words.
+// candidate is disabled.  lds: KS_LDS_WORDS 64-bit words; lkey, lidx: P each.
 __device__ __forceinline__ int64_t relax_db(int64_t P, int nsrc, const double* const* maps, double tol, uint32_t* bits, int32_t* ev,
-                            uint64_t* lds, SelScratch& sh) {
+                            uint64_t* lkey, int32_t* lidx, uint64_t* lds, SelScratch& sh) {
   __shared__ int64_t lenj[IQ_MAX_AUX + 2];
   const int64_t nwd = (P + 31) / 32;
   // enabled patterns = finite entries of D; all zero when none is finite and nonzero (relaxation.jl:7-11)
   const auto* dg = iq_glob(maps[0]);
   int64_t cf = 0, cz = 0;
-  for (int64_t i0 = threadIdx.x; i0 < P; i0 += 8 * FB) {  // eight loads in flight
-    double x[8];
+  for (int64_t i0 = threadIdx.x; i0 < P; i0 += KS_U * FB) {
+    double x[KS_U];
 #pragma unroll
-    for (int k = 0; k < 8; k++) x[k] = i0 + k * FB < P ? dg[i0 + k * FB] : __builtin_inf();
+    for (int k = 0; k < KS_U; k++) x[k] = i0 + k * FB < P ? dg[i0 + k * FB] : __builtin_inf();
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
+    for (int k = 0; k < KS_U; k++) {
       const bool fin = !__builtin_isinf(x[k]);
       cf += fin;
       cz += fin && x[k] != 0.0;
@@ -790,32 +947,24 @@ __device__ __forceinline__ int64_t relax_db(int64_t P, int nsrc, const double* c
   const int64_t dbsize = allzero ? nen : (int64_t)ceil(tol * (double)nen);
   if (dbsize <= 0) return -1;  // tol outside (0, 1]: the loop would never end
   if (threadIdx.x < IQ_MAX_AUX + 2) lenj[threadIdx.x] = 0;
-  {
-    uint64_t tv;
-    int64_t ti;
-    blk_kth_key(maps[0], P, dbsize, lds, sh, &tv, &ti);
-    blk_prefix_bits(maps[0], P, tv, ti, bits);
-  }
   __syncthreads();
   double frac = 0.1 * ((double)dbsize / (double)nen);
   int64_t cnt = dbsize;
   for (;;) {
     const int64_t softdbsize = (int64_t)ceil(frac * (double)nen);
     cnt = dbsize;
-    for (int j = 1; j < nsrc; j++) {
+    for (int j = 0; j < nsrc; j++) {
       // the prefix only grows (frac does); an unchanged length keeps its bitmap
-      if (softdbsize != lenj[j]) {
-        uint64_t tv = 0;
-        int64_t ti = -1;  // empty prefix
-        if (softdbsize > 0) blk_kth_key(maps[j], P, softdbsize < P ? softdbsize : P, lds, sh, &tv, &ti);
-        blk_prefix_bits(maps[j], P, tv, ti, bits + j * nwd);
-        __syncthreads();
-        if (threadIdx.x == 0) lenj[j] = softdbsize;
+      const int64_t len = j == 0 ? dbsize : softdbsize;
+      if (len != lenj[j]) {
+        blk_prefix(maps[j], P, len < P ? len : P, bits + j * nwd, lkey, lidx, lds, sh);
+        if (threadIdx.x == 0) lenj[j] = len;
       }
+      if (j == 0) continue;
       int64_t lc = 0;
       for (int64_t w = threadIdx.x; w < nwd; w += FB) {
-        uint32_t x = bits[w];
-        for (int k = 1; k <= j; k++) x &= bits[k * nwd + w];
+        uint32_t x = ks_word(bits + w);
+        for (int k = 1; k <= j; k++) x &= ks_word(bits + k * nwd + w);
         lc += __builtin_popcount(x);
       }
       cnt = blk_sum_i64(lc, sh);
@@ -829,15 +978,15 @@ __device__ __forceinline__ int64_t relax_db(int64_t P, int nsrc, const double* c
   const int64_t w0 = threadIdx.x * per, w1 = (w0 + per < nwd) ? w0 + per : nwd;
   int64_t lc = 0;
   for (int64_t w = w0; w < w1; w++) {
-    uint32_t x = bits[w];
-    for (int k = 1; k < nsrc; k++) x &= bits[k * nwd + w];
+    uint32_t x = ks_word(bits + w);
+    for (int k = 1; k < nsrc; k++) x &= ks_word(bits + k * nwd + w);
     lc += __builtin_popcount(x);
   }
   int64_t nev;
   int64_t off = blk_excl_scan(lc, &nev, sh);
   for (int64_t w = w0; w < w1; w++) {
-    uint32_t x = bits[w];
-    for (int k = 1; k < nsrc; k++) x &= bits[k * nwd + w];
+    uint32_t x = ks_word(bits + w);
+    for (int k = 1; k < nsrc; k++) x &= ks_word(bits + k * nwd + w);
     while (x) {
       int b = __builtin_ctz(x);
       x &= x - 1;
@@ -878,7 +1027,9 @@ k_relax_finalize(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
   nsrc = sh.flag;
   __syncthreads();
   int32_t* ev = D->ev + slot * g.P;
-  const int64_t nev = relax_db(g.P, nsrc, mp, D->tol, D->bits + slot * D->nmap * D->nw32, ev, (uint64_t*)sv, sh);
+  // list scratch: the slot's key and superset lists (used later, by the ranks of a large database)
+  const int64_t nev = relax_db(g.P, nsrc, mp, D->tol, D->bits + slot * D->nmap * D->nw32, ev,
+                               (uint64_t*)(D->rkey + slot * 2 * g.P), D->sup + slot * g.P, (uint64_t*)sv, sh);
   if (nev < 0) {
     if (threadIdx.x == 0) { set_err(D->err, IQ_KERR_NOCAND); *o.pick = -2; }
     return;
@@ -923,10 +1074,11 @@ k_band_pick_host(const double* __restrict__ Dm, int64_t n, double tol, int32_t* 
 
 extern "C" __global__ void __launch_bounds__(FB)
 k_relax_host(int64_t P, int nsrc, const double* const* __restrict__ maps, double tol, uint32_t* __restrict__ bits,
-             int32_t* __restrict__ ev, int64_t* __restrict__ count, int32_t* __restrict__ err) {
+             int32_t* __restrict__ ev, uint64_t* __restrict__ lkey, int32_t* __restrict__ lidx, int64_t* __restrict__ count,
+             int32_t* __restrict__ err) {
   __shared__ SelScratch sh;
   __shared__ uint64_t ks[KS_LDS_WORDS];
-  const int64_t n = relax_db(P, nsrc, maps, tol, bits, ev, ks, sh);
+  const int64_t n = relax_db(P, nsrc, maps, tol, bits, ev, lkey, lidx, ks, sh);
   if (threadIdx.x == 0) {
     if (n < 0) set_err(err, IQ_KERR_NOCAND);
     *count = n < 0 ? 0 : n;
