@@ -990,11 +990,9 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
     IqMask& m = pl->masks[mi];
     double* a2 = pl->mem.alloc<double>(g.P);
     if (pl->dtype == IQ_F32)
-      hipLaunchKernelGGL((k_exact_map<float, 2>), dim3(nblk(g.P, 256)), dim3(256), 0, s, (const float*)H.ti, g,
-                         H.toff + m.off, (const double*)nullptr, m.V, (const double*)nullptr, a2);
+      launch_exact_map<float, 2>(s, (const float*)H.ti, g, H.toff + m.off, nullptr, m.V, a2);
     else
-      hipLaunchKernelGGL((k_exact_map<double, 2>), dim3(nblk(g.P, 256)), dim3(256), 0, s, (const double*)H.ti, g,
-                         H.toff + m.off, (const double*)nullptr, m.V, (const double*)nullptr, a2);
+      launch_exact_map<double, 2>(s, (const double*)H.ti, g, H.toff + m.off, nullptr, m.V, a2);
     HCL();
     // padded to whole 32-candidate chunks of the bank scan, the pad NaN
     const int64_t P32 = (g.P + 31) / 32 * 32;
@@ -1145,8 +1143,7 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
       double* at = pl->mem.upload(d->auxti[a], (size_t)tivox, s);
       auxtip.push_back(at);
       double* a2 = pl->mem.alloc<double>(g.P);
-      hipLaunchKernelGGL((k_exact_map<double, 2>), dim3(nblk(g.P, 256)), dim3(256), 0, s, (const double*)at, g,
-                         H.toff + full_off, (const double*)nullptr, g.tilevox, (const double*)nullptr, a2);
+      launch_exact_map<double, 2>(s, at, g, H.toff + full_off, nullptr, g.tilevox, a2);
       HCL();
       a2sp.push_back(a2);
     }
@@ -2888,32 +2885,24 @@ int iq_fastdistance(iq_ctx* ctx, const void* img, int img_dtype, const int64_t i
       if (kdims[d] <= 0 || g.dist[d] <= 0) bad(IQ_ERR_ARG, "kernel larger than image");
     hipStream_t s = ctx->stream;
     DMem m;
-    std::vector<int32_t> tv, to;
+    std::vector<int32_t> to;
+    std::vector<double> kv;
     for (int32_t t = 0; t < g.tilevox; t++)
       if (!weights || weights[t]) {
         int x = t % g.tile[0], y = (t / g.tile[0]) % g.tile[1], z = t / (g.tile[0] * g.tile[1]);
-        tv.push_back(t);
+        kv.push_back(kern[t]);
         to.push_back((int32_t)(x + (int64_t)g.ti[0] * (y + (int64_t)g.ti[1] * z)));
       }
-    int V = (int)tv.size();
+    const int V = (int)to.size();
     int64_t ni = idims[0] * idims[1] * idims[2];
     const size_t esz = img_dtype == IQ_F32 ? 4 : 8;
     char* di = m.alloc<char>(ni * esz);
     HC(hipMemcpyAsync(di, img, ni * esz, hipMemcpyHostToDevice, s));
-    double* dk = m.upload(kern, (size_t)g.tilevox, s);
-    int32_t* dtv = m.upload(tv.data(), tv.size(), s);
+    double* dk = m.upload(kv.data(), kv.size(), s);
     int32_t* dto = m.upload(to.data(), to.size(), s);
-    double* kv = m.alloc<double>(std::max(V, 1));
-    double* b2 = m.alloc<double>(1);
     double* dout = m.alloc<double>(g.P);
-    hipLaunchKernelGGL(k_gather_b2, dim3(1), dim3(256), 0, s, (const double*)dk, (const int32_t*)dtv, V, kv, b2);
-    HCL();
-    if (img_dtype == IQ_F32)
-      hipLaunchKernelGGL((k_exact_map<float, 0>), dim3(nblk(g.P, 256)), dim3(256), 0, s, (const float*)di, g,
-                         (const int32_t*)dto, (const double*)kv, V, (const double*)b2, dout);
-    else
-      hipLaunchKernelGGL((k_exact_map<double, 0>), dim3(nblk(g.P, 256)), dim3(256), 0, s, (const double*)di, g,
-                         (const int32_t*)dto, (const double*)kv, V, (const double*)b2, dout);
+    if (img_dtype == IQ_F32) launch_exact_map<float, 0>(s, (const float*)di, g, dto, dk, V, dout);
+    else launch_exact_map<double, 0>(s, (const double*)di, g, dto, dk, V, dout);
     HCL();
     HC(hipMemcpyAsync(out, dout, g.P * sizeof(double), hipMemcpyDeviceToHost, s));
     HC(hipStreamSynchronize(s));
