@@ -550,9 +550,19 @@ dim3 scan_grid(const iq_plan* pl, int nq, int nw) {
   const int ntile = (nq + 31) / 32;
   return dim3(nblk(g.dist[0], 32), nblk(g.dist[1], 4 * nw), (unsigned)(g.dist[2] * ntile));
 }
-void launch_scan_mfma(iq_plan* pl, const IqQuery* q, int nq, int nw, hipStream_t s) {
-  hipLaunchKernelGGL((pl->mfma_split ? k_scan_mfma<true> : k_scan_mfma<false>),
-                     scan_grid(pl, nq, nw), dim3(64 * nw), pl->lds_nw[nw], s, (const IqDev*)pl->dd, q, nq, pl->mfma_gerr,
+// Whether a scan lists the candidates near its bound (k_scan_mfma) instead of
+// storing every one's: from one and a half rounds of resident wavefronts (12 a
+// compute unit).  Scan and selection, stored and listed, in us by wavefronts:
+// 16: 22, 25; 264: 21, 21; 2,898: 80, 75; 3,300: 95, 99; 6,072: 135, 120;
+// 6,600: 191, 157; 13,200: 339, 262; 52,800: 1,388, 996.
+bool scan_lists(const iq_plan* pl, int nq, int nw) {
+  const dim3 gr = scan_grid(pl, nq, nw);
+  return (int64_t)gr.x * gr.y * gr.z * nw >= 256 * 18;
+}
+void launch_scan_mfma(iq_plan* pl, const IqQuery* q, int nq, int nw, bool list, hipStream_t s) {
+  const auto k = pl->mfma_split ? (list ? k_scan_mfma<true, true> : k_scan_mfma<true, false>)
+                                : (list ? k_scan_mfma<false, true> : k_scan_mfma<false, false>);
+  hipLaunchKernelGGL(k, scan_grid(pl, nq, nw), dim3(64 * nw), pl->lds_nw[nw], s, (const IqDev*)pl->dd, q, nq, pl->mfma_gerr,
                      pl->kofs_nw[nw], pl->exact_int ? 1 : 0);
   HCL();
 }
@@ -605,7 +615,7 @@ void tune_scan(iq_plan* pl) {
       float tot = 0.0f;
       for (int rep = 0; rep < 4; rep++) {
         if (rep == 1) HC(hipEventRecord(a, s));
-        launch_scan_mfma(pl, dq, nq, nw, s);
+        launch_scan_mfma(pl, dq, nq, nw, scan_lists(pl, nq, nw), s);
       }
       HC(hipEventRecord(b, s));
       HC(hipEventSynchronize(b));
@@ -1121,8 +1131,9 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
         for (size_t m = 0; m < hmasks.size(); m++) std::memcpy(&mb[m * g.tilevox], hmasks[m].bits.data(), g.tilevox);
         H.maskbits = pl->mem.upload(mb.data(), mb.size(), s);
         if (lmax > 64 * 1024) {
-          HC(hipFuncSetAttribute((const void*)k_scan_mfma<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lmax));
-          HC(hipFuncSetAttribute((const void*)k_scan_mfma<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lmax));
+          for (const void* k : {(const void*)k_scan_mfma<true, false>, (const void*)k_scan_mfma<true, true>,
+                                (const void*)k_scan_mfma<false, false>, (const void*)k_scan_mfma<false, true>})
+            HC(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lmax));
         }
       }
     }
@@ -1232,6 +1243,7 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
   H.sup = pl->mem.alloc<int32_t>((size_t)NS * P);
   H.rkey = pl->mem.alloc<unsigned long long>((size_t)NS * 2 * P);
   H.nsup = pl->mem.alloc<int32_t>(NS);
+  H.ncand = pl->mem.alloc<int32_t>(NS);
   H.sd = pl->mem.alloc<double>((size_t)NS * IQ_SORT_MAX);
   H.si = pl->mem.alloc<int32_t>((size_t)NS * IQ_SORT_MAX);
   H.s1 = pl->mem.alloc<double>((size_t)NS * (nw64 + 1));
@@ -1444,6 +1456,7 @@ void run_batch(iq_plan* pl, const IqQuery* hq, const IqQuery* q, int nq, bool ha
   if (has_plain && nfull > 0) {
     // the full scan over the batch's first nf queries
     const int nf = nfull;
+    bool list = false;
     if (pl->fast) {
       if (pl->prof && pl->prof_used + 2 > (int64_t)pl->prof_ev.size()) {
         hipEvent_t a, b;
@@ -1470,7 +1483,8 @@ void run_batch(iq_plan* pl, const IqQuery* hq, const IqQuery* q, int nq, bool ha
           pl->prof_mflop += (double)grid.x * rows * g.dist[2] * ntile * pl->hd.ktab.nstep * (pl->mfma_split ? 3.0 : 1.0) *
                             (2.0 * 32 * 32 * 16);
         }
-        launch_scan_mfma(pl, q, nf, nw, s);
+        list = scan_lists(pl, nf, nw);
+        launch_scan_mfma(pl, q, nf, nw, list, s);
       } else {
         if (pl->prof) HC(hipEventRecord(pl->prof_ev[pl->prof_used], s));
         launch_scan_batch(pl, q, nf, s);
@@ -1487,7 +1501,10 @@ void run_batch(iq_plan* pl, const IqQuery* hq, const IqQuery* q, int nq, bool ha
         pl->prof_flop += f;
       }
       const bool exact = pl->mfma && pl->exact_int;
-      hipLaunchKernelGGL(k_band_select, dim3(nblk(P, 256 * SEL_PT), nf), dim3(256), 0, s, D, q, exact ? 1 : 0);
+      if (list)
+        hipLaunchKernelGGL(k_list_select, dim3(std::min(nblk(P, 256), 32u), nf), dim3(256), 0, s, D, q, exact ? 1 : 0);
+      else
+        hipLaunchKernelGGL(k_band_select, dim3(nblk(P, 256 * SEL_PT), nf), dim3(256), 0, s, D, q, exact ? 1 : 0);
       HCL();
       if (!exact) launch_recheck(pl, q, nf, s);
     } else {
@@ -2277,7 +2294,7 @@ void harvest_queries(iq_plan* pl, std::vector<std::pair<int32_t, int32_t>> pool,
       const int ntile = (nq + 31) / 32;
       hipLaunchKernelGGL(k_mfma_bprep, dim3(pl->hd.ktab.nstep, ntile), dim3(64), 0, s, D, (const IqQuery*)dq, nq);
       const int nw = pl->mfma_nw_forced ? pl->mfma_nw : pl->nw_tiles[ntile > 1 ? 2 : 1];
-      launch_scan_mfma(pl, dq, nq, nw, s);
+      launch_scan_mfma(pl, dq, nq, nw, false, s);
     } else {
       launch_scan_batch(pl, dq, nq, s);
     }

@@ -208,6 +208,7 @@ struct IqDev {
   int32_t* sup;                            // superset list, P per slot (then ranks of a large band)
   unsigned long long* rkey;                // 2P per slot: radix keys of a large band (then its weights)
   int32_t* nsup;
+  int32_t* ncand;                          // entries of the MFMA scan's list (lo32: bounds, band: candidates)
   double* sd;                              // IQ_SORT_MAX per slot (band distances, then weights)
   int32_t* si;                             // IQ_SORT_MAX per slot (ranks)
   double* s1;        int64_t s1_stride;

@@ -155,6 +155,7 @@ __device__ __forceinline__ void query_prep_body(const IqDev* __restrict__ D, con
       D->gmin_hi[slot] = 0x7f800000u;
       D->gmin64[slot] = 0x7ff0000000000000ull;
       D->nsup[slot] = 0;
+      D->ncand[slot] = 0;
     }
   } else if (src == 1) {
     if (!q.multi || q.rep != q.slot || !st.hard) return;
@@ -672,12 +673,24 @@ __device__ __forceinline__ void scan_frags(const uint32_t* lw, int at, const int
   }
 }
 
-template <bool SPLIT>
+// LIST: candidates within the band of the least upper bound known so far are
+// listed (lo32: bounds, band: candidates, ncand: how many; every member of the
+// final superset is among them) in place of a store of every bound, which no
+// line is whole in (the lanes hold a candidate of 32 queries each) and the
+// selection reads again.  The bound returned by the atomic is waited for: read
+// ahead of the k-steps it is too old (facies scans took a tenth longer).  Scan
+// and selection over 402,075 windows of 24x24x6 codes, 512 queries: 1,388 us
+// with the store, 996 with the list; 64 queries 191 and 157.  In a launch of
+// one round no group knows another's bound and the wait is not covered: 32
+// queries 95 and 99, one query tile in 4 groups 22 and 25 (scan_lists draws
+// the line).
+template <bool SPLIT, bool LIST>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 k_scan_mfma(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int nq, double gerr,
             const int32_t* __restrict__ kofs_tab, int exact) {
   extern __shared__ __align__(16) uint32_t lw[];
-  __shared__ float red[4][32];
+  __shared__ float red[4][32], thr[32];
+  __shared__ int sslot[32];
   const IqGeo& g = D->g;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int row = lane & 31, kb = lane >> 5;
@@ -784,6 +797,8 @@ k_scan_mfma(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int nq,
   float lmin = __builtin_inff();
   bool live = false;
   int64_t slot = 0;
+  float B = 0.0f, sB = 0.0f, k1 = 0.0f, k2 = 0.0f, tiny2 = 0.0f;
+  const float* a2p = nullptr;
   if (qi < nq) {
     const IqQuery q = qs[qi];
     const IqStep& st = D->steps[q.step];
@@ -799,74 +814,141 @@ k_scan_mfma(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int nq,
       // terms are doubled to cover the rounding of d -/+ e, and lo / hi are
       // pushed outward by 2^-20.  A2 = NaN marks a disabled window.
       const IqMask& m = D->masks[st.mask];
-      const auto a2f = iq_glob(D->a2f[m.a2]);
-      const float B = (float)D->b2[slot * (2 + D->naux)];
-      const float sB = __builtin_amdgcn_sqrtf(fmaxf(B, 0x1p-100f)) * (1.0f + 0x1p-19f);
+      a2p = D->a2f[m.a2];
+      B = (float)D->b2[slot * (2 + D->naux)];
+      sB = __builtin_amdgcn_sqrtf(fmaxf(B, 0x1p-100f)) * (1.0f + 0x1p-19f);
       const double V = (double)m.V;
       const double g64 = V * 0x1p-53 / (1.0 - V * 0x1p-53);
       const float gs2 = (float)((gerr + g64) * (1.0 + 0x1p-10)) * 2.0f * (1.0f + 0x1p-10f);
       const float u32 = 0x1p-24f;
-      const float tiny2 = 2.0f * (float)(1e3 * V * 0x1p-125);
+      tiny2 = 2.0f * (float)(1e3 * V * 0x1p-125);
       // e = gs2 S + 2 (8 u32 ((A + B) + 2 S)) + tiny2, regrouped as
       // S (gs2 + 32 u32) + 16 u32 (A + B) + tiny2 and evaluated by two fmas:
       // fewer roundings than the plain sum, each within the margins above
-      const float k1 = gs2 + 32.0f * u32, k2 = 16.0f * u32;
-      const auto lo_out = iq_globw(D->lo32 + slot * g.P);
+      k1 = gs2 + 32.0f * u32;
+      k2 = 16.0f * u32;
+    }
+  }
+  // (integer codes: every operand and result is an integer below 2^24)
+  const auto bound = [&](auto codes, float a, float ab, float& hi) {
+    const float d = __builtin_fabsf(__builtin_fmaf(-2.0f, ab, a) + B);  // 2 ab is exact
+    float lo = d;
+    hi = d;
+    if constexpr (!codes.value) {
+      const float S = __builtin_amdgcn_sqrtf(fmaxf(a, 0x1p-100f)) * sB;
+      const float e = __builtin_fmaf(S, k1, __builtin_fmaf(a + B, k2, tiny2));
+      lo = fmaxf(d - e, 0.0f) * (1.0f - 0x1p-20f);
+      hi = (d + e) * (1.0f + 0x1p-20f);
+    }
+    if (a != a) lo = hi = __builtin_inff();
+    return lo;
+  };
+  const auto bounds = [&](auto codes) {
+    const auto a2f = iq_glob(a2p);
+    const auto lo_out = iq_globw(D->lo32 + slot * g.P);
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int cy = cy0 + 4 * w + i;
-        if (cy >= d1) break;  // uniform per wavefront
-        const int64_t rb = (int64_t)d0 * (cy + (int64_t)d1 * cz) + cx0 + 4 * kb;
-        const int xl = d0 - cx0 - 4 * kb;  // candidates of this row left to the lane
-        float A[16];
+    for (int i = 0; i < 4; i++) {
+      const int cy = cy0 + 4 * w + i;
+      if (cy >= d1) break;  // uniform per wavefront
+      const int64_t rb = (int64_t)d0 * (cy + (int64_t)d1 * cz) + cx0 + 4 * kb;
+      const int xl = d0 - cx0 - 4 * kb;  // candidates of this row left to the lane
+      float A[16];
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-          const int ox = 8 * (v >> 2) + (v & 3);
-          A[v] = a2f[ox < xl ? rb + ox : rb - 4 * kb];
-        }
-        if (exact) {  // uniform: every operand and result is an integer below 2^24
+      for (int v = 0; v < 16; v++) {
+        const int ox = 8 * (v >> 2) + (v & 3);
+        A[v] = a2f[ox < xl ? rb + ox : rb - 4 * kb];
+      }
 #pragma unroll
-          for (int v = 0; v < 16; v++) {
-            const int ox = 8 * (v >> 2) + (v & 3);
-            float d = __builtin_fabsf(__builtin_fmaf(-2.0f, acc[i][v], A[v]) + B);
-            if (A[v] != A[v]) d = __builtin_inff();
-            if (ox < xl) {
-              lo_out[rb + ox] = d;
-              lmin = fminf(lmin, d);
-            }
-          }
-          continue;
-        }
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-          const int ox = 8 * (v >> 2) + (v & 3);
-          const float a = A[v];
-          const float d = __builtin_fabsf(__builtin_fmaf(-2.0f, acc[i][v], a) + B);  // 2 acc is exact
-          const float S = __builtin_amdgcn_sqrtf(fmaxf(a, 0x1p-100f)) * sB;
-          const float e = __builtin_fmaf(S, k1, __builtin_fmaf(a + B, k2, tiny2));
-          float lo = fmaxf(d - e, 0.0f) * (1.0f - 0x1p-20f);
-          float hi = (d + e) * (1.0f + 0x1p-20f);
-          if (a != a) lo = hi = __builtin_inff();
-          if (ox < xl) {
-            lo_out[rb + ox] = lo;
-            lmin = fminf(lmin, hi);
-          }
+      for (int v = 0; v < 16; v++) {
+        const int ox = 8 * (v >> 2) + (v & 3);
+        float hi;
+        const float lo = bound(codes, A[v], acc[i][v], hi);
+        if (LIST) acc[i][v] = ox < xl ? lo : __builtin_inff();
+        if (ox < xl) {
+          if (!LIST) lo_out[rb + ox] = lo;
+          lmin = fminf(lmin, hi);
         }
       }
     }
+  };
+  if (live) {
+    if (exact) bounds(std::true_type());
+    else bounds(std::false_type());
+  }
+  if constexpr (!LIST) {
+    lmin = fminf(lmin, __shfl_xor(lmin, 32));
+    if (kb == 0) red[w][row] = lmin;
+    __syncthreads();
+    if (w == 0 && kb == 0 && live) {
+      float m = red[0][row];
+      for (int i = 1; i < nw; i++) m = fminf(m, red[i][row]);
+      atomicMin(&D->gmin_hi[slot], __float_as_uint(m));
+    }
+    return;
   }
   lmin = fminf(lmin, __shfl_xor(lmin, 32));
-  if (kb == 0) red[w][row] = lmin;
+  if (kb == 0) {
+    red[w][row] = lmin;
+    if (w == 0) sslot[row] = live ? (int)slot : -1;
+  }
   __syncthreads();
-  if (w == 0 && kb == 0 && live) {
-    float m = red[0][row];
-    for (int i = 1; i < nw; i++) m = fminf(m, red[i][row]);
-    atomicMin(&D->gmin_hi[slot], __float_as_uint(m));
+  // this group's share of the queries' bitmaps is cleared for the selection
+  {
+    const int nwg = (int)(gridDim.x * gridDim.y) * g.dist[2];
+    const int fb = (int)blockIdx.x + (int)gridDim.x * ((int)blockIdx.y + (int)gridDim.y * cz);
+    const int per = (int)((D->nw64 + nwg - 1) / nwg);
+    for (int i = threadIdx.x; i < 32 * per; i += NT) {
+      const int64_t wd = (int64_t)fb * per + i % per;
+      const int sl = sslot[i / per];
+      if (sl >= 0 && wd < D->nw64) D->bitmap[sl * D->nw64 + wd] = 0ull;
+    }
+  }
+  if (w == 0 && kb == 0) {
+    float T = -1.0f;
+    if (live) {
+      float m = red[0][row];
+      for (int i = 1; i < nw; i++) m = fminf(m, red[i][row]);
+      const float U = fminf(m, __uint_as_float(atomicMin(&D->gmin_hi[slot], __float_as_uint(m))));
+      T = fminf(iq_f32_up((1.0 + D->tol) * (double)U), __FLT_MAX__);
+    }
+    thr[row] = T;
+  }
+  __syncthreads();
+  const float T = thr[row];
+  const int rows = d1 - cy0 - 4 * w;  // uniform per wavefront
+  int n = 0;
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    if (i < rows)
+#pragma unroll
+      for (int v = 0; v < 16; v++) n += acc[i][v] <= T;
+  if (__ballot(live && n > 0) == 0ull) return;  // uniform per wavefront
+  if (!live) n = 0;
+  const int other = __shfl_xor(n, 32);
+  int base = 0;
+  if (kb == 0 && n + other > 0) base = atomicAdd(&D->ncand[slot], n + other);
+  base = __shfl(base, row) + (kb ? other : 0);
+  if (n == 0) return;
+  const auto lo_out = iq_globw(D->lo32 + slot * g.P);
+  const auto id_out = iq_globw(D->band + slot * g.P);
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    if (i >= rows) break;
+    const int64_t r0 = (int64_t)d0 * (cy0 + 4 * w + i + (int64_t)d1 * cz) + cx0 + 4 * kb;
+#pragma unroll
+    for (int v = 0; v < 16; v++)
+      if (acc[i][v] <= T && base < g.P) {
+        lo_out[base] = acc[i][v];
+        id_out[base] = (int32_t)(r0 + 8 * (v >> 2) + (v & 3));
+        base++;
+      }
   }
 }
 
-template __global__ void k_scan_mfma<true>(const IqDev*, const IqQuery*, int, double, const int32_t*, int);
-template __global__ void k_scan_mfma<false>(const IqDev*, const IqQuery*, int, double, const int32_t*, int);
+template __global__ void k_scan_mfma<true, false>(const IqDev*, const IqQuery*, int, double, const int32_t*, int);
+template __global__ void k_scan_mfma<true, true>(const IqDev*, const IqQuery*, int, double, const int32_t*, int);
+template __global__ void k_scan_mfma<false, false>(const IqDev*, const IqQuery*, int, double, const int32_t*, int);
+template __global__ void k_scan_mfma<false, true>(const IqDev*, const IqQuery*, int, double, const int32_t*, int);
 
 #define IQ_SCAN_INST(R, LX, LY, LZ) \
   template __global__ void k_scan_f32<R, LX, LY, LZ>(const IqDev*, const IqQuery*, int);
@@ -927,6 +1009,41 @@ k_band_select(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int e
       if (exact) D->dexact[slot * P + c] = (double)v[j];
     }
     base += __popcll(bal[j]);
+  }
+}
+
+// The same superset from the list of the MFMA scan, whose bitmap is cleared.
+// Grid: (list blocks, query).
+__global__ void __launch_bounds__(256)
+k_list_select(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int exact) {
+  const IqQuery q = qs[blockIdx.y];
+  const IqStep& st = D->steps[q.step];
+  if (q.multi || st.mask < 0) return;
+  const int64_t P = D->g.P;
+  const int64_t slot = q.slot;
+  const double U = (double)__uint_as_float(D->gmin_hi[slot]);
+  const float Tf = iq_f32_up((1.0 + D->tol) * U);
+  if (exact && blockIdx.x == 0 && threadIdx.x == 0)
+    D->gmin64[slot] = (unsigned long long)__double_as_longlong(U);
+  const int64_t cnt = D->ncand[slot], n = cnt < P ? cnt : P;
+  const auto lo = iq_glob(D->lo32 + slot * P);
+  const auto id = iq_glob(D->band + slot * P);
+  const int lane = threadIdx.x & 63;
+  for (int64_t i0 = (int64_t)blockIdx.x * 256 + (threadIdx.x & ~63); i0 < n; i0 += (int64_t)gridDim.x * 256) {
+    const int64_t i = i0 + lane;
+    const float v = i < n ? lo[i] : __builtin_inff();
+    const int32_t c = i < n ? id[i] : 0;
+    const bool in = i < n && v <= Tf;
+    const unsigned long long bal = __ballot(in);
+    if (!bal) continue;  // uniform per wavefront
+    int base = 0;
+    if (lane == 0) base = atomicAdd(&D->nsup[slot], __popcll(bal));
+    base = __builtin_amdgcn_readfirstlane(base);
+    if (in) {
+      D->sup[slot * P + base + __popcll(bal & ((1ull << lane) - 1ull))] = c;
+      atomicOr(&D->bitmap[slot * D->nw64 + (c >> 6)], 1ull << (c & 63));
+      if (exact) D->dexact[slot * P + c] = (double)v;
+    }
   }
 }
 
