@@ -743,11 +743,16 @@ k_scan_mfma(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int nq,
 #pragma unroll
     for (int c = 0; c < 4; c++) off[c] = 2 * c % kbx.cy + ry * (2 * c / kbx.cy);
     // k-steps: B fragments and chunk offsets are loaded ahead, one step for
-    // split data (a step's twelve MFMAs cover the load: two ahead measured 8 %
-    // slower), two for the four MFMAs of bf16-exact data (6 % faster);
+    // split data (a step's twelve MFMAs cover the load; two ahead are no
+    // faster), AHEAD for the four MFMAs of bf16-exact data.  There the loads
+    // past the box's end repeat its last step's: with a test the wait of the
+    // loop's head is for every load in flight.  Scans of codes with the list,
+    // 126 launches on average: 522 us two ahead with the test, 479 four ahead
+    // without, 457 eight (with the store, one round: 93, 88, 96);
     // consecutive MFMAs use different accumulators
-    iq_u32x4 bh[2], bl[2];
-    int ko[2];
+    constexpr int AHEAD = SPLIT ? 2 : (LIST ? 8 : 4);
+    iq_u32x4 bh[AHEAD], bl[AHEAD];
+    int ko[AHEAD];
     auto fetch = [&](int u, int step) {
       bh[u] = bhp[(int64_t)step * 64];
       if (SPLIT) bl[u] = blp[(int64_t)step * 64];
@@ -771,9 +776,8 @@ k_scan_mfma(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int nq,
       }
     };
     const int s0 = kbx.s0, s1 = kbx.s1;
-    if (s0 < s1) fetch(SPLIT ? 1 : 0, s0);
-    if (!SPLIT && s0 + 1 < s1) fetch(1, s0 + 1);
     if constexpr (SPLIT) {
+      if (s0 < s1) fetch(1, s0);
       for (int step = s0; step < s1; step++) {
         bh[0] = bh[1];
         bl[0] = bl[1];
@@ -782,14 +786,19 @@ k_scan_mfma(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int nq,
         mfmas(0);
       }
     } else {
+#pragma unroll
+      for (int u = 0; u < AHEAD; u++) fetch(u, s0 + u < s1 ? s0 + u : s1 - 1);
       int step = s0;
-      for (; step + 1 < s1; step += 2) {
-        mfmas(0);
-        if (step + 2 < s1) fetch(0, step + 2);
-        mfmas(1);
-        if (step + 3 < s1) fetch(1, step + 3);
+      for (; step + AHEAD <= s1; step += AHEAD) {
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) {
+          mfmas(u);
+          fetch(u, step + AHEAD + u < s1 ? step + AHEAD + u : s1 - 1);
+        }
       }
-      if (step < s1) mfmas(0);
+#pragma unroll
+      for (int u = 0; u + 1 < AHEAD; u++)
+        if (step + u < s1) mfmas(u);
     }
   }
   // epilogue: lane holds C[row'][col] for col = lane % 32 (its query)
