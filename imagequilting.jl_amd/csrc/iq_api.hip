@@ -551,13 +551,13 @@ dim3 scan_grid(const iq_plan* pl, int nq, int nw) {
   return dim3(nblk(g.dist[0], 32), nblk(g.dist[1], 4 * nw), (unsigned)(g.dist[2] * ntile));
 }
 // Whether a scan lists the candidates near its bound (k_scan_mfma) instead of
-// storing every one's: from one and a half rounds of resident wavefronts (12 a
-// compute unit).  Scan and selection, stored and listed, in us by wavefronts:
-// 16: 22, 25; 264: 21, 21; 2,898: 80, 75; 3,300: 95, 99; 6,072: 135, 120;
-// 6,600: 191, 157; 13,200: 339, 262; 52,800: 1,388, 996.
+// storing every one's: from a wavefront per compute unit.  Scan and selection,
+// stored and listed, in us by wavefronts: 16: 22, 25; 252: 34, 34; 264: 21, 20;
+// 504: 35, 34; 2,160: 68, 65; 2,898: 80, 74; 3,300: 89, 87; 5,796: 136, 119;
+// 6,600: 184, 136; 13,200: 319, 222; 52,800: 1,306, 864.
 bool scan_lists(const iq_plan* pl, int nq, int nw) {
   const dim3 gr = scan_grid(pl, nq, nw);
-  return (int64_t)gr.x * gr.y * gr.z * nw >= 256 * 18;
+  return (int64_t)gr.x * gr.y * gr.z * nw >= 256;
 }
 void launch_scan_mfma(iq_plan* pl, const IqQuery* q, int nq, int nw, bool list, hipStream_t s) {
   const auto k = pl->mfma_split ? (list ? k_scan_mfma<true, true> : k_scan_mfma<true, false>)

@@ -679,11 +679,11 @@ __device__ __forceinline__ void scan_frags(const uint32_t* lw, int at, const int
 // line is whole in (the lanes hold a candidate of 32 queries each) and the
 // selection reads again.  The bound returned by the atomic is waited for: read
 // ahead of the k-steps it is too old (facies scans took a tenth longer).  Scan
-// and selection over 402,075 windows of 24x24x6 codes, 512 queries: 1,388 us
-// with the store, 996 with the list; 64 queries 191 and 157.  In a launch of
-// one round no group knows another's bound and the wait is not covered: 32
-// queries 95 and 99, one query tile in 4 groups 22 and 25 (scan_lists draws
-// the line).
+// and selection over 402,075 windows of 24x24x6 codes, 512 queries: 1,306 us
+// with the store, 864 with the list; 64 queries 184 and 136, 32 queries 89 and
+// 87.  In a launch of a few groups no group knows another's bound and the wait
+// is not covered: one query tile in 4 groups 22 and 25 (scan_lists draws the
+// line).
 template <bool SPLIT, bool LIST>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 k_scan_mfma(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int nq, double gerr,
