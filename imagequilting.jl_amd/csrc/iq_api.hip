@@ -328,11 +328,24 @@ bool fits_f32(const double* v, int64_t n) {
 // E[t^2] <= 32 Var[t] the interval stays near 2^-9 of them and the superset
 // near the band.  Beyond that (and for a constant image) the exhaustive FP64
 // map stays: its time does not depend on the values.
-bool scan_takes_rounded(const double* v, int64_t n) {
-  double s1 = 0.0, s2 = 0.0;
+// The interval also has terms that do not scale with the values (operands
+// clamped up to 2^-100, some V 2^-114 for what underflows), which exceed every
+// distance of an image below about 1e-17.  So `scale` is the power of two that
+// takes the largest magnitude to [1, 2) (1 where it is larger): multiplying
+// by it is exact, and the interval keeps its share of the distances.  (64x64x32
+// image times 1e-18, tile 14x14x5: every window rechecked and 162 ms a
+// realization without it, 8 windows and 10 ms with it.)
+bool scan_takes_rounded(const double* v, int64_t n, double* scale) {
+  double mx = 0.0;
   for (int64_t i = 0; i < n; i++) {
     const double x = v[i];
     if (!(std::fabs(x) <= 0x1p50) || (x != 0.0 && std::fabs(x) < 0x1p-100)) return false;
+    mx = std::max(mx, std::fabs(x));
+  }
+  *scale = mx > 0.0 && mx < 1.0 ? std::ldexp(1.0, -std::ilogb(mx)) : 1.0;
+  double s1 = 0.0, s2 = 0.0;
+  for (int64_t i = 0; i < n; i++) {
+    const double x = v[i] * *scale;
     s1 += x;
     s2 += x * x;
   }
@@ -944,6 +957,7 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
   // ---- training image
   IqDev& H = pl->hd;
   H.g = g;
+  H.scan_s = H.scan_s2 = 1.0;
   const double* tid = (const double*)d->ti;
   const float* tif = (const float*)d->ti;
   int vmax = 0;  // voxels of the largest overlap mask
@@ -960,10 +974,12 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
   } else {
     H.ti = pl->mem.upload(tid, tivox, s);
     pl->fast = fits_f32(tid, tivox);
-    if (!pl->fast) pl->fast = pl->rounded = scan_takes_rounded(tid, tivox);
+    if (!pl->fast) pl->fast = pl->rounded = scan_takes_rounded(tid, tivox, &H.scan_s);
+    if (!pl->rounded) H.scan_s = 1.0;
+    H.scan_s2 = H.scan_s * H.scan_s;
     if (pl->fast) {
       std::vector<float> t32((size_t)tivox);
-      for (int64_t i = 0; i < tivox; i++) t32[i] = (float)tid[i];
+      for (int64_t i = 0; i < tivox; i++) t32[i] = (float)(tid[i] * H.scan_s);
       exact16 = bf16_exact(t32.data(), tivox);
       pl->exact_int = exact16 && !pl->rounded && exact_codes(t32.data(), tivox, vmax);
       H.ti32 = pl->mem.upload(t32.data(), tivox, s);
@@ -1009,7 +1025,7 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
     float* a2f = pl->mem.alloc<float>(P32);
     if (P32 > g.P) HC(hipMemsetAsync(a2f + g.P, 0xff, (P32 - g.P) * sizeof(float), s));
     hipLaunchKernelGGL(k_a2_f32, dim3(std::min<int64_t>(nblk(g.P, 256), 4096)), dim3(256), 0, s, (const double*)a2,
-                       (const uint8_t*)H.disabled, g.P, a2f);
+                       (const uint8_t*)H.disabled, g.P, H.scan_s2, a2f);
     HCL();
     m.a2 = (int32_t)a2ptr.size();
     a2ptr.push_back(a2);

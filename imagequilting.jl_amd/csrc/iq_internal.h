@@ -170,7 +170,8 @@ struct IqReal {
 struct IqDev {
   IqGeo g;
   const void* ti;
-  const float* ti32;
+  const float* ti32;     // FP32 image of the scans; Float64 images that are rounded for them: times scan_s
+  double scan_s, scan_s2;  // power of two the MFMA scan's operands are taken times, and its square (1 but for rounded images)
   int32_t ti_f32;
   int32_t naux;
   double tol;

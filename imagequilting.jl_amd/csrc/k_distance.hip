@@ -570,7 +570,7 @@ __device__ __forceinline__ void mfma_bprep_body(const IqDev* __restrict__ D, con
         } else {
           const double* sim64 = (const double*)D->sims + R.sim_off;
 #pragma unroll
-          for (int e = 0; e < 8; e++) v[e] = (float)sim64[gi[e]];
+          for (int e = 0; e < 8; e++) v[e] = (float)(sim64[gi[e]] * D->scan_s);
         }
 #pragma unroll
         for (int e = 0; e < 8; e++) {
@@ -612,12 +612,13 @@ k_prep_bprep(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int nq
 template __global__ void k_prep_bprep<float>(const IqDev*, const IqQuery*, int, int);
 template __global__ void k_prep_bprep<double>(const IqDev*, const IqQuery*, int, int);
 
-// FP32 copy of an A2 map for the scan's interval bound; NaN marks a disabled
-// window (an A2 that overflows FP32 becomes +inf and stays a candidate)
+// FP32 copy of an A2 map, times s2 (scan_s2), for the scan's interval bound;
+// NaN marks a disabled window (an A2 that overflows FP32 becomes +inf and
+// stays a candidate)
 __global__ void __launch_bounds__(256)
-k_a2_f32(const double* __restrict__ a2, const uint8_t* __restrict__ disabled, int64_t P, float* __restrict__ out) {
+k_a2_f32(const double* __restrict__ a2, const uint8_t* __restrict__ disabled, int64_t P, double s2, float* __restrict__ out) {
   for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < P; c += (int64_t)gridDim.x * 256)
-    out[c] = disabled[c] ? __builtin_nanf("") : (float)a2[c];
+    out[c] = disabled[c] ? __builtin_nanf("") : (float)(a2[c] * s2);
 }
 
 // The image in the words the scan stages, y fastest: word (y, x, z) holds the
@@ -821,10 +822,12 @@ k_scan_mfma(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int nq,
       // evaluation of d as well as the oracle's own FP64 rounding.  The main
       // term carries a 2^-10 margin for its own FP32 evaluation, the small
       // terms are doubled to cover the rounding of d -/+ e, and lo / hi are
-      // pushed outward by 2^-20.  A2 = NaN marks a disabled window.
+      // pushed outward by 2^-20.  A2 = NaN marks a disabled window.  All of it
+      // is in units of scan_s2: the operands are a power of two times the
+      // image's values, so its distances are that power squared times these.
       const IqMask& m = D->masks[st.mask];
       a2p = D->a2f[m.a2];
-      B = (float)D->b2[slot * (2 + D->naux)];
+      B = (float)(D->b2[slot * (2 + D->naux)] * D->scan_s2);
       sB = __builtin_amdgcn_sqrtf(fmaxf(B, 0x1p-100f)) * (1.0f + 0x1p-19f);
       const double V = (double)m.V;
       const double g64 = V * 0x1p-53 / (1.0 - V * 0x1p-53);
