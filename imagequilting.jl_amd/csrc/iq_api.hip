@@ -1361,10 +1361,19 @@ void launch_mscan(iq_plan* pl, const IqQuery* q, const int4* tiles, int ntiles, 
 }
 
 // exact FP64 recheck of the band supersets of a batch: with a lane per
-// member, or (IQHIP_RECHECK=groups) a wavefront per member
+// member, or (IQHIP_RECHECK=groups) a wavefront per member.  The superset of a
+// rounded image may be wide for its values alone (white noise, tol 1: 63,207
+// of 72,828 windows), where the exhaustive map would have had every compute
+// unit at work; so its grid holds a wavefront per RCL_MPW candidates, up to
+// RCL_WIDE wavefronts.  That image took 248 ms a realization with RCL_GROUPS a
+// query, 182, 167 and 164 with 2,048, 4,096 and 8,192 wavefronts, and 174 with
+// the exhaustive map on the vector units; wavefronts without a member leave at
+// once (supersets of 8 members: 14.4 ms with any of these).
 void launch_recheck(iq_plan* pl, const IqQuery* q, int nq, hipStream_t s) {
+  unsigned groups = RCL_GROUPS;
+  if (pl->rounded) groups = std::max<unsigned>(groups, std::min<unsigned>(nblk(pl->geo.P, RCL_MPW), RCL_WIDE / nq));
   if (pl->hd.rc_lanes == 0)
-    hipLaunchKernelGGL(k_band_recheck_lanes, dim3(nq, RCL_GROUPS), dim3(64), 0, s, (const IqDev*)pl->dd, q);
+    hipLaunchKernelGGL(k_band_recheck_lanes, dim3(nq, groups), dim3(64), 0, s, (const IqDev*)pl->dd, q);
   else
     hipLaunchKernelGGL(k_band_recheck, dim3(nq, RC_GROUPS), dim3(256), 0, s, (const IqDev*)pl->dd, q);
   HCL();

@@ -1265,8 +1265,9 @@ k_band_recheck(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
 // the scalar cache does not hold a query's 38 KB, and every 16 chain steps
 // waited on a scalar load.)  Few members per wavefront keep
 // one round of loads per block and many wavefronts per query.
-// Grid: (query, RCL_GROUPS wavefronts), members beyond loop.
+// Grid: (query, RCL_GROUPS wavefronts or more), members beyond loop.
 #define RCL_GROUPS 32
+#define RCL_WIDE 8192  // most wavefronts of a launch over a rounded image
 #define RCL_MPW 16
 template <typename E>
 __device__ __forceinline__ double rcl_chain(const IqDev* __restrict__ D, int64_t base, const int32_t* __restrict__ toff,

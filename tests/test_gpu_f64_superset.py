@@ -30,3 +30,10 @@ def test_small_values_match_oracle(scale):
     T = _smooth(np.random.default_rng(72), (33, 29, 13), 5, np.float64) * scale
     print("scale", scale, flush=True)
     _compare(T, (9, 10, 5), (30, 37, 14), overlap=(0.25, 0.25, 0.25))
+
+
+@pytest.mark.parametrize("nreal", [1, 70])  # a wavefront per 16 candidates, and fewer
+def test_wide_superset_matches_oracle(nreal):
+    T = np.random.default_rng(73).standard_normal((60, 57))
+    print("white noise, realizations", nreal, flush=True)
+    _compare(T, (8, 8), (20, 22), overlap=(0.25, 0.25), tol=1.0, nreal=nreal)
