@@ -1116,7 +1116,7 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
         rym = std::max(rym, iq_scan_ry(H.ktab.box[b].wyr, 4));
       }
       const int64_t nwords = tivox + (int64_t)g.ti[1] * (rxm + 33) + rym + 64;
-      if ((pl->lds_nw[2] || pl->lds_nw[4]) && nwords < (1ll << 31)) {
+      if (lmax > 0 && nwords < (1ll << 31)) {  // some group size fits (one is tried when it is forced)
         pl->mfma = true;
         pl->mfma_lds = lmax;
         pl->mfma_split = split;
