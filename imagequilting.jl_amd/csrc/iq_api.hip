@@ -580,11 +580,16 @@ void launch_scan_mfma(iq_plan* pl, const IqQuery* q, int nq, int nw, bool list, 
   HCL();
 }
 
-// Scan autotuner: the MFMA scan's group size (2 or 4 wavefronts) is measured
+// Scan autotuner: the MFMA scan's group size (2, 3 or 4 wavefronts) is measured
 // on the plan itself.  A batch of the plan's own masked steps (32 queries,
 // then up to 64 as the slots allow) is prepared once; each group size runs one
-// warm-up and three timed launches; the faster is kept per tile count.  The
-// choice changes speed only: both sizes compute the same bounds.
+// warm-up and three timed launches (the least counts: a launch timed by itself
+// may be late); the fastest size is kept per tile count.  What a listing scan
+// writes depends on the bound and the list it starts from, so both are reset
+// before every launch, outside the time taken (an image of ties, 301,806
+// windows, 32 queries: 64 us a launch on a list that is full already, 123 with
+// two wavefronts and 156 with four as a run launches it).  The choice changes
+// speed only: all sizes compute the same bounds.
 template <typename T>
 void tune_scan(iq_plan* pl) {
   const int nwa[3] = {2, 3, 4};
@@ -613,9 +618,8 @@ void tune_scan(iq_plan* pl) {
   const IqQuery* dq = pl->mem.upload(hq.data(), hq.size(), s);
   hipLaunchKernelGGL((k_fill<T>), dim3(1024), dim3(256), 0, s, (T*)pl->hd.sims, pl->nvox, (T)0);
   HCL();
-  hipEvent_t a, b;
-  HC(hipEventCreate(&a));
-  HC(hipEventCreate(&b));
+  hipEvent_t ev[6];
+  for (hipEvent_t& e : ev) HC(hipEventCreate(&e));
   for (int ntile = 1; ntile <= 2; ntile++) {
     const int nq = ntile == 1 ? 32 : (int)hq.size();  // two tiles: every prepared query (33 to 64)
     if (ntile == 2 && nq <= 32) break;
@@ -625,22 +629,29 @@ void tune_scan(iq_plan* pl) {
     HCL();
     float best = 1e30f;
     for (int nw : nwa) {
-      float tot = 0.0f;
-      for (int rep = 0; rep < 4; rep++) {
-        if (rep == 1) HC(hipEventRecord(a, s));
-        launch_scan_mfma(pl, dq, nq, nw, scan_lists(pl, nq, nw), s);
+      const bool list = scan_lists(pl, nq, nw);
+      for (int rep = -1; rep < 3; rep++) {
+        if (list) {  // the queries' slots are 0 to nq - 1
+          hipLaunchKernelGGL(k_scan_reset, dim3(1), dim3(64), 0, s, D, nq);
+          HCL();
+        }
+        if (rep >= 0) HC(hipEventRecord(ev[2 * rep], s));
+        launch_scan_mfma(pl, dq, nq, nw, list, s);
+        if (rep >= 0) HC(hipEventRecord(ev[2 * rep + 1], s));
       }
-      HC(hipEventRecord(b, s));
-      HC(hipEventSynchronize(b));
-      HC(hipEventElapsedTime(&tot, a, b));
-      const float us = tot * 1e3f / 3.0f;
+      HC(hipEventSynchronize(ev[5]));
+      float us = 1e30f;
+      for (int rep = 0; rep < 3; rep++) {
+        float ms = 0.0f;
+        HC(hipEventElapsedTime(&ms, ev[2 * rep], ev[2 * rep + 1]));
+        us = std::min(us, ms * 1e3f);
+      }
       pl->tune_us[ntile][nw] = us;
       if (us < best) { best = us; pl->nw_tiles[ntile] = nw; }
     }
   }
   if ((int)hq.size() <= 32) pl->nw_tiles[2] = pl->nw_tiles[1];
-  HC(hipEventDestroy(a));
-  HC(hipEventDestroy(b));
+  for (hipEvent_t e : ev) HC(hipEventDestroy(e));
 }
 
 // Voxel lists of the exact maps (k_maps.hip): every mask's, then the whole

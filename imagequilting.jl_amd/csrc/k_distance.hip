@@ -962,6 +962,14 @@ template __global__ void k_scan_mfma<true, true>(const IqDev*, const IqQuery*, i
 template __global__ void k_scan_mfma<false, false>(const IqDev*, const IqQuery*, int, double, const int32_t*, int);
 template __global__ void k_scan_mfma<false, true>(const IqDev*, const IqQuery*, int, double, const int32_t*, int);
 
+// What a listing scan of the slots [0, n) starts from, as k_query_prep leaves it.
+__global__ void __launch_bounds__(64) k_scan_reset(const IqDev* __restrict__ D, int n) {
+  for (int i = threadIdx.x; i < n; i += 64) {
+    D->gmin_hi[i] = 0x7f800000u;
+    D->ncand[i] = 0;
+  }
+}
+
 #define IQ_SCAN_INST(R, LX, LY, LZ) \
   template __global__ void k_scan_f32<R, LX, LY, LZ>(const IqDev*, const IqQuery*, int);
 IQ_SCAN_INST(4, 8, 8, 4)
