@@ -60,13 +60,15 @@ namespace {
 // Work-items of a cut launch whose largest slab has n interior nodes: a lane
 // per node up to `most` (CUT_TEAM_MAX, or 512 under IQHIP_CUT_TEAM), then two
 // or three nodes a lane (1,536 nodes on 1,024 lanes, half of them with two: 489
-// us per 96 slabs, against 548 us on 768 lanes with two each) ...
+// us per 96 slabs, against 548 us on 768 lanes with two each), and all lanes
+// over the global scratch of slabs beyond CUT_REG_MAX (4,800 nodes: 15.1 ms a
+// launch on 256 lanes, 8.7 on 512, 5.4 on 1,024) ...
 int cut_team(int64_t n, int most = CUT_TEAM_MAX) {
-  if (n > CUT_REG_MAX) return 256;
   return (int)std::min<int64_t>(most, std::max<int64_t>(64, (n + 63) / 64 * 64));
 }
 
-// ... and its nodes a lane (0: node state in global scratch)
+// ... and its nodes a lane (0: three, and global scratch for the slabs beyond
+// CUT_REG_MAX)
 int cut_npt(int64_t n, int team) { return n > CUT_REG_MAX ? 0 : (int)std::max<int64_t>(1, (n + team - 1) / team); }
 
 template <typename T>
@@ -89,7 +91,7 @@ auto cut_host_kernel(int npt) {
 }
 
 // LDS bytes of one slab's cut of n interior nodes (register-resident form;
-// larger slabs keep their state in global scratch)
+// slabs beyond CUT_REG_MAX keep their state in global scratch)
 size_t cut_lds_bytes(int64_t n) {
   return n <= CUT_REG_MAX ? (size_t)((n + 63) / 64 * 64) * CUT_FAST_NODE_BYTES : 0;
 }
@@ -469,7 +471,7 @@ struct iq_plan {
   int64_t dm_cap = 0;
   double* mpack = nullptr;   // their query values in fragment order (one batch at a time)
   int64_t mpack_cap = 0;
-  int cut_npt = 1;         // interior nodes a lane of a cut (0: global scratch)
+  int cut_npt = 1;         // interior nodes a lane of a cut (0: three, and slabs in global scratch)
   int cut_team = 256;      // work-items of a cut (IQHIP_CUT_TEAM=512: at most 512)
   int max_nslab = 1;       // most min cuts of any step: the cut launches' grid width
   bool cut_wave = false;   // every slab fits the one-wavefront cut
@@ -1223,14 +1225,16 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
   const int nmap = 2 + pl->naux;
   int kmax = 4;
   for (const IqMask& m : pl->masks) kmax = std::max(kmax, m.kbox);
-  int64_t maxn = 0;
+  int64_t maxn = 0, maxreg = 0;  // largest slab, largest of at most CUT_REG_MAX nodes
   for (const IqStep& st : pl->steps)
     for (int q = 0; q < st.nslab; q++) {
       const IqSlab& sl = st.slab[q];
-      maxn = std::max(maxn, (int64_t)sl.sz[0] * sl.sz[1] * sl.sz[2] / sl.sz[sl.dim] * std::max(0, sl.sz[sl.dim] - 2));
+      const int64_t n = (int64_t)sl.sz[0] * sl.sz[1] * sl.sz[2] / sl.sz[sl.dim] * std::max(0, sl.sz[sl.dim] - 2);
+      maxn = std::max(maxn, n);
+      if (n <= CUT_REG_MAX) maxreg = std::max(maxreg, n);
     }
   for (const IqStep& st : pl->steps) pl->max_nslab = std::max(pl->max_nslab, st.ncut);
-  pl->cut_lds_max = cut_lds_bytes(maxn);
+  pl->cut_lds_max = cut_lds_bytes(maxreg);
   pl->cut_wave = maxn <= CUT_WAVE_MAX;
   const char* et = std::getenv("IQHIP_CUT_TEAM");
   pl->cut_team = cut_team(maxn, et && std::atoi(et) == 512 && maxn <= 3 * 512 ? 512 : CUT_TEAM_MAX);

@@ -652,19 +652,18 @@ __device__ __forceinline__ void cut_slab_fast(const SlabView<T>& A, const SlabVi
 }
 
 // One slab by the whole workgroup (a multiple of 64 work-items): up to NPT
-// register-resident nodes a lane; NPT = 0: node state in global scratch.
+// register-resident nodes a lane; NPT = 0: up to three on CUT_TEAM_MAX lanes,
+// node state in global scratch beyond CUT_REG_MAX nodes.
 template <typename T, int NPT>
 __device__ __forceinline__ void cut_dispatch(const SlabView<T>& A, const SlabView<T>& B, const int s[3], int dim, uint8_t side,
                                              uint8_t* out, char* lds, char* gmem, int32_t* err, int64_t* rounds) {
   const int n = s[0] * s[1] * s[2] / s[dim] * (s[dim] > 2 ? s[dim] - 2 : 0);
   const int team = (int)blockDim.x;
-  if constexpr (NPT == 0) {
-    cut_slab<T>(A, B, s, dim, side, out, gmem, err, rounds);
-  } else {
-    if (NPT >= 3 && n > 2 * team) cut_slab_fast<T, 3, false>(A, B, s, dim, side, out, lds, err, rounds);
-    else if (NPT >= 2 && n > team) cut_slab_fast<T, 2, false>(A, B, s, dim, side, out, lds, err, rounds);
-    else cut_slab_fast<T, 1, false>(A, B, s, dim, side, out, lds, err, rounds);
-  }
+  constexpr int MOST = NPT == 0 ? 3 : NPT;
+  if (NPT == 0 && n > CUT_REG_MAX) cut_slab<T>(A, B, s, dim, side, out, gmem, err, rounds);
+  else if (MOST >= 3 && n > 2 * team) cut_slab_fast<T, 3, false>(A, B, s, dim, side, out, lds, err, rounds);
+  else if (MOST >= 2 && n > team) cut_slab_fast<T, 2, false>(A, B, s, dim, side, out, lds, err, rounds);
+  else cut_slab_fast<T, 1, false>(A, B, s, dim, side, out, lds, err, rounds);
 }
 
 // The slab blockIdx.x of query blockIdx.y: A = the realization's grid over the
@@ -699,6 +698,8 @@ __device__ __forceinline__ bool cut_views(const IqDev* __restrict__ D, const IqQ
 
 // Batched cut: grid (slab, query).  The workgroup has a lane for every node of
 // the plan's largest slab, up to CUT_TEAM_MAX, then two or three nodes a lane.
+// In a plan with slabs beyond CUT_REG_MAX nodes (NPT = 0) each slab takes the
+// form of its own size.
 template <typename T, int NPT>
 __global__ void __launch_bounds__(CUT_TEAM_MAX)
 k_graphcut(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
@@ -749,7 +750,8 @@ k_graphcut_host(const T* __restrict__ a, const T* __restrict__ b, int s0, int s1
   SlabView<T> A, B;
   A.base = a; A.st[0] = 1; A.st[1] = s0; A.st[2] = (int64_t)s0 * s1;
   B.base = b; B.st[0] = 1; B.st[1] = s0; B.st[2] = (int64_t)s0 * s1;
-  cut_dispatch<T, NPT>(A, B, s, dim, (uint8_t)0, out, cut_lds, gmem, err, nullptr);
+  if constexpr (NPT == 0) cut_slab<T>(A, B, s, dim, (uint8_t)0, out, gmem, err, nullptr);  // launched for such a slab alone
+  else cut_dispatch<T, NPT>(A, B, s, dim, (uint8_t)0, out, cut_lds, gmem, err, nullptr);
 }
 
 #define CUT_HOST_INST(T)                                                                                         \
