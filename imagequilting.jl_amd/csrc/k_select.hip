@@ -658,13 +658,47 @@ __device__ __forceinline__ int blk_find_bin(const uint32_t* hist, int nb, int64_
   return bin;
 }
 
+// Index of the r-th value of the map, in index order, whose bits are pv (there
+// are at least r): a counting pass per wavefront segment, then a walk of the
+// one segment that holds it.
+__device__ __forceinline__ int64_t blk_kth_tie(const double* __restrict__ map, int64_t P, uint64_t pv, int64_t r, SelScratch& sh) {
+  const auto* mg = iq_glob(map);
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t seg = (P + NW * 64 - 1) / (NW * 64) * 64;
+  const int64_t a = wv * seg, e = a + seg < P ? a + seg : P;
+  int64_t c = 0;
+  for (int64_t base = a; base < e; base += 64) {
+    const int64_t i = base + lane;
+    c += __popcll(__ballot(i < e && f64_bits(mg[i]) == pv));
+  }
+  const int64_t ex = blk_excl_scan(lane == 0 ? c : 0, nullptr, sh);
+  const int64_t pre = __shfl(ex, 0);
+  if (pre < r && r <= pre + c) {
+    int64_t need = r - pre;
+    for (int64_t base = a; base < e; base += 64) {
+      const int64_t i = base + lane;
+      uint64_t b = __ballot(i < e && f64_bits(mg[i]) == pv);
+      const int k = __popcll(b);
+      if (need <= k) {
+        for (int64_t t = 1; t < need; t++) b &= b - 1;
+        if (lane == 0) sh.result = base + __ffsll((unsigned long long)b) - 1;
+        break;
+      }
+      need -= k;
+    }
+  }
+  __syncthreads();
+  const int64_t ti = sh.result;
+  __syncthreads();
+  return ti;
+}
+
 // The m-th smallest (1 <= m <= P) pair (bits(map[i]), i) over i in [0, P).
 // Radix digits of 11 bits over the value bits, each a histogram pass over
 // the map restricted to the prefix fixed so far, until the bin holding rank
 // m has at most KS_CAP members; those are compacted into LDS and ranked
 // pairwise.  When the whole value is fixed with more than KS_CAP ties, the
-// m-th is found by index order directly (a counting pass per wavefront
-// segment, then a walk of the one segment that holds it).
+// m-th is found by index order directly (blk_kth_tie).
 __device__ __forceinline__ void blk_kth_key(const double* __restrict__ map, int64_t P, int64_t m, uint64_t* lds, SelScratch& sh,
                             uint64_t* tv, int64_t* ti) {
   uint32_t* hist = (uint32_t*)lds;
@@ -707,35 +741,8 @@ __device__ __forceinline__ void blk_kth_key(const double* __restrict__ map, int6
     known += w;
   }
   if (cnt > KS_CAP) {
-    // value fixed (pv), rank r among its ties in index order
-    const int wv = threadIdx.x >> 6;
-    const int64_t seg = (P + NW * 64 - 1) / (NW * 64) * 64;
-    const int64_t a = wv * seg, e = a + seg < P ? a + seg : P;
-    int64_t c = 0;
-    for (int64_t base = a; base < e; base += 64) {
-      const int64_t i = base + lane;
-      c += __popcll(__ballot(i < e && f64_bits(mg[i]) == pv));
-    }
-    const int64_t ex = blk_excl_scan(lane == 0 ? c : 0, nullptr, sh);
-    const int64_t pre = __shfl(ex, 0);
-    if (pre < r && r <= pre + c) {
-      int64_t need = r - pre;
-      for (int64_t base = a; base < e; base += 64) {
-        const int64_t i = base + lane;
-        uint64_t b = __ballot(i < e && f64_bits(mg[i]) == pv);
-        const int k = __popcll(b);
-        if (need <= k) {
-          for (int64_t t = 1; t < need; t++) b &= b - 1;
-          if (lane == 0) sh.result = base + __ffsll((unsigned long long)b) - 1;
-          break;
-        }
-        need -= k;
-      }
-    }
-    __syncthreads();
     *tv = pv;
-    *ti = sh.result;
-    __syncthreads();
+    *ti = blk_kth_tie(map, P, pv, r, sh);
     return;
   }
   // compact the bin's members into LDS (any order), then rank them pairwise
@@ -815,8 +822,13 @@ __device__ __forceinline__ void blk_prefix_bits(const double* __restrict__ map, 
 // statistic is found in the list, whose members then get their bits.  The
 // passes over the maps are what the relaxation costs, and the radix selection
 // takes four: 336 queries of 3 maps of 216,225 values took 988 us that way,
-// 684 us this way (the bits and the list are what a pass writes).  False, with
-// the bits to be written again, when the bracket missed or too many members tie.
+// 684 us this way (the bits and the list are what a pass writes).  Ties (maps of
+// codes, of few hard points) are known by value from the list, or from one
+// counting pass where the bracket is a single value; the radix selection goes
+// through every digit of them.  Two maps of 216,225 values in 40 and 3 levels:
+// 1,021 us with the selection after a pass in vain, 863 with it alone, 449
+// this way.  False, with the bits to be written again, when the bracket missed
+// or is one value of the top words only.
 __device__ __forceinline__ bool blk_prefix_sampled(const double* __restrict__ map, int64_t P, int64_t m, uint32_t* __restrict__ bits,
                                                    uint64_t* __restrict__ lkey, int32_t* __restrict__ lidx, uint64_t* lds,
                                                    SelScratch& sh) {
@@ -849,7 +861,35 @@ __device__ __forceinline__ bool blk_prefix_sampled(const double* __restrict__ ma
     br[side] = pv;
   }
   const uint32_t lo = br[0], hi = br[1];
-  if (lo == hi) return false;  // tied values
+  if (lo == hi) {
+    // tied: how many are below, how many in the bracket, do those agree in
+    // their low words (ones and zeros: bits set in any, bits clear in any)?
+    int64_t nlo = 0, nin = 0;
+    uint32_t ones = 0, zeros = 0;
+    for (int64_t i0 = threadIdx.x; i0 < P; i0 += KS_U * FB) {
+      uint64_t v[KS_U];
+#pragma unroll
+      for (int k = 0; k < KS_U; k++) v[k] = i0 + k * FB < P ? f64_bits(mg[i0 + k * FB]) : ~0ull;
+#pragma unroll
+      for (int k = 0; k < KS_U; k++) {
+        const uint32_t h = (uint32_t)(v[k] >> 32);
+        const bool in = h == lo && i0 + k * FB < P;
+        nlo += h < lo;
+        nin += in;
+        ones |= in ? (uint32_t)v[k] : 0u;
+        zeros |= in ? ~(uint32_t)v[k] : 0u;
+      }
+    }
+    const int64_t r = m - blk_sum_i64(nlo, sh), n = blk_sum_i64(nin, sh);
+    const uint64_t b = blk_or_u64((uint64_t)zeros << 32 | ones, sh);
+    ones = (uint32_t)b;
+    zeros = (uint32_t)(b >> 32);
+    if (r < 1 || r > n || (ones & zeros)) return false;
+    const uint64_t tv = (uint64_t)lo << 32 | ones;
+    blk_prefix_bits(map, P, tv, blk_kth_tie(map, P, tv, r, sh), bits);
+    __syncthreads();
+    return true;
+  }
   if (threadIdx.x == 0) sh.flag = 0;
   __syncthreads();
   const int64_t nwd = (P + 31) / 32;
@@ -894,7 +934,7 @@ __device__ __forceinline__ bool blk_prefix_sampled(const double* __restrict__ ma
   // the r-th smallest (value, index) pair of the list
   uint64_t* cv = lds + 1024;
   uint32_t* ci = (uint32_t*)(lds + 1024 + KS_CAP);
-  int known = lo == hi ? 32 : __builtin_clz(lo ^ hi);  // leading bits the bracket fixes
+  int known = __builtin_clz(lo ^ hi);  // leading bits the bracket fixes
   uint64_t hm = known ? ~0ull << (64 - known) : 0ull, pv = ((uint64_t)lo << 32) & hm;
   while (known < 64 && cnt > KS_CAP) {
     const int w = 64 - known >= 11 ? 11 : 64 - known;
@@ -912,7 +952,11 @@ __device__ __forceinline__ bool blk_prefix_sampled(const double* __restrict__ ma
     hm |= (uint64_t)dm << sft;
     known += w;
   }
-  if (cnt > KS_CAP) { __syncthreads(); return false; }
+  if (cnt > KS_CAP) {  // so many ties: the value is known, the index is found in the map
+    blk_prefix_bits(map, P, pv, blk_kth_tie(map, P, pv, r, sh), bits);
+    __syncthreads();
+    return true;
+  }
   if (threadIdx.x == 0) sh.flag = 0;
   __syncthreads();
   for (int i = threadIdx.x; i < n; i += FB) {
