@@ -624,10 +624,11 @@ k_band_finalize(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int
 // ---------------------------------------------------------------------------
 #define KS_CAP 512          // bins this small are ranked pairwise in LDS
 #define KS_SAMPLE 4096      // sample of a map from which its order statistic is bracketed
-// Smaller maps are selected without a sample: two sources take 66 us without
-// and 79 us with it at 16,384 values, 112 and 107 at 32,768, 150 and 105 at
-// 65,536, 544 and 289 at 262,144.
-#define KS_MIN 32768
+// Smaller maps are selected without a sample.  A realization with one soft
+// variable, ms without and with the sample by candidates: 40,000: 7.7, 8.9;
+// 44,944: 8.2, 9.2; 49,729: 8.6, 9.2; 55,696: 8.9, 8.9; 59,536: 9.4, 8.9; 71,824:
+// 10.3, 9.4; 147,456: 16.6, 13.5; 262,144: 26.0, 19.5.
+#define KS_MIN 57344
 #define KS_U 8              // loads in flight per work-item in the passes over a map
 #define KS_LDS_WORDS 3072   // 64-bit LDS words: histogram 2048 x u32, then the sample (u32), or KS_CAP values and indices
 

@@ -33,3 +33,15 @@ def test_tied_prefix_sets_match_oracle(ctx, n, kind):
         print(n, kind, tol, flush=True)
         got = iqhip.relaxation(D, [A], tol, ctx=ctx)
         assert np.array_equal(got, iqref.relaxation(D, [A], tol)), tol
+
+
+@pytest.mark.parametrize("n", [57343, 57344, 57377])  # below, at and above the smallest sampled map
+@pytest.mark.parametrize("kind", ["continuous", "levels"])
+def test_smallest_sampled_map_matches_oracle(ctx, n, kind):
+    rng = np.random.default_rng(n)
+    D, A = rng.random(n), rng.random(n)
+    if kind == "levels":
+        D, A = np.floor(D * 30), np.floor(A * 4)
+    for tol in (1e-4, 0.1, 0.999):
+        print(n, kind, tol, flush=True)
+        assert np.array_equal(iqhip.relaxation(D, [A], tol, ctx=ctx), iqref.relaxation(D, [A], tol)), tol
