@@ -435,7 +435,6 @@ struct iq_plan {
   bool fast = false;
   bool exact_int = false;  // the MFMA scan's FP32 distances are exact (integer codes)
   bool rounded = false;  // fast, on the FP32 rounding of Float64 data (MFMA scan only)
-  bool hard = false;
   bool any_multi = false;
   std::vector<IqStep> steps;
   std::vector<IqMask> masks;
@@ -463,7 +462,7 @@ struct iq_plan {
   int4* dt = nullptr;    // shortlist tiles (all batches of a run)
   int64_t dt_cap = 0;
   size_t cut_lds_max = 0;
-  size_t hard_lds = 0;     // LDS of the tiled hard-data maps (0: gathering kernel)
+  size_t hard_lds = 0;     // LDS of the tiled hard-data maps
   int hard_bx = 16;        // candidate block width of the tiled maps (32 or 16; 16 rows)
   size_t maps_lds = 0;     // LDS of the exact maps (k_maps_mfma), 0: not used by the plan
   int maps_steps = 0;      // most steps of any voxel list
@@ -846,12 +845,10 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
   std::vector<HostMask> hmasks;
   std::vector<int32_t> htvox;
   std::vector<int64_t> mask_uses;
-  pl->hard = false;
   for (int gi = 0; gi < ngrid; gi++) {
   const iq_plan_desc* e = &descs[gi];
   HostGrid& G = pl->grids[gi];
   G.step0 = (int64_t)pl->steps.size();
-  if (e->hardgrid) pl->hard = true;
   const int64_t nt = G.ntiles[0] * G.ntiles[1] * G.ntiles[2];
   std::vector<uint8_t> pasted((size_t)nt, 0);
   for (int64_t i = 0; i < e->npath; i++) {
@@ -1290,20 +1287,24 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
   H.nw32 = nw32;
   if (pl->any_multi || (!pl->fast && !hmasks.empty())) build_map_lists(pl, tvox, full_off, s);
   if (pl->any_multi) {
-    // hard-data maps: tiled when some tile holds at least HARD_TILED points
-    // and the candidate block's training-image region fits in LDS (voxel lists
-    // as offsets into the staged region, read as scalar loads; candidate
-    // blocks of 32 x 16 where the region fits, else 16 x 16;
-    // IQHIP_MAPS_BX=16 forces the narrow blocks)
+    // hard-data maps: the tiles from hard_min points on are made by the tiled
+    // kernel where the candidate block's training-image region fits in LDS
+    // (voxel lists as offsets into the staged region, read as scalar loads;
+    // candidate blocks of 32 x 16 where the region fits, else 16 x 16).
+    // IQHIP_MAPS_BX=32 or 16 makes every tile's there, in blocks of at most
+    // that width.
     int hmax = 0;
     for (const IqStep& st : pl->steps) hmax = std::max(hmax, st.hcnt);
     const char* ebx = std::getenv("IQHIP_MAPS_BX");
+    H.hard_min = INT32_MAX;
     for (int bx : {32, 16}) {
       if (bx == 32 && ebx && std::atoi(ebx) == 16) continue;
-      if (hmax < HARD_TILED && !ebx) break;
       const int RX = bx + g.tile[0] - 1, RY = 16 + g.tile[1] - 1;
       const size_t need = (size_t)RX * RY * g.tile[2] * 8;
       if (need > 150 * 1024 || htvox.empty()) continue;
+      const int from = ebx ? 1 : (int)((need / 8 * HARD_TILED + bx * 16 - 1) / (bx * 16));
+      if (hmax < from) break;
+      H.hard_min = from;
       std::vector<int32_t> rh(htvox.size());
       for (size_t i = 0; i < htvox.size(); i++) {
         const int t = htvox[i], x = t % g.tile[0], y = (t / g.tile[0]) % g.tile[1], z = t / (g.tile[0] * g.tile[1]);
@@ -1559,12 +1560,19 @@ void run_batch(iq_plan* pl, const IqQuery* hq, const IqQuery* q, int nq, bool ha
     }
   }
   if (has_multi) {
-    if (pl->hard) {
+    bool few = false, many = false;  // steps by the kernel that makes their hard map
+    for (int i = 0; i < nq; i++) {
+      const IqStep& st = pl->steps[hq[i].step];
+      if (hq[i].multi && st.hard) (st.hcnt < pl->hd.hard_min ? few : many) = true;
+    }
+    if (few) {
+      hipLaunchKernelGGL(k_hard_maps, dim3(nblk(P, 256), nq), dim3(256), 0, s, D, q);
+      HCL();
+    }
+    if (many) {
       const int bx = pl->hard_bx;
       const unsigned nb = nblk(g.dist[0], bx) * nblk(g.dist[1], 16) * (unsigned)g.dist[2];
-      if (pl->hard_lds == 0)
-        hipLaunchKernelGGL(k_hard_maps, dim3(nblk(P, 256), nq), dim3(256), 0, s, D, q);
-      else if (bx == 32)
+      if (bx == 32)
         hipLaunchKernelGGL((k_hard_maps_tiled<32, 16>), dim3(nb, nq), dim3(512), pl->hard_lds, s, D, q);
       else
         hipLaunchKernelGGL((k_hard_maps_tiled<16, 16>), dim3(nb, nq), dim3(256), pl->hard_lds, s, D, q);

@@ -185,6 +185,7 @@ struct IqDev {
   const int32_t* htvox;  // hard voxels per step
   const int32_t* htoff;
   const int32_t* rhtvox;  // htvox entries as offsets into the tiled hard map's staged region
+  int32_t hard_min;       // hard points of a tile from which its map is made by the tiled kernel
   int32_t full_off;
   const double* const* a2maps;
   const float* const* a2f;  // FP32 copies of a2maps, NaN where the window is disabled

@@ -1385,12 +1385,17 @@ k_band_recheck_lanes(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs
 // windows from the image: a tile usually holds a handful of points, for which
 // staging its windows' region (k_hard_maps_tiled) costs more than it saves.
 // ---------------------------------------------------------------------------
-#define HARD_TILED 48  // hard points of a tile from which the plan uses the tiled form
+// A tile takes the tiled form from this many hard points for every voxel that
+// form stages per candidate.  Gathered and tiled, us a launch by points of a
+// tile: 225 x 225 candidates, tile 32 x 32 (5.8 voxels): 8: 10, 14; 24: 15, 14;
+// 32: 19, 15; 128: 55, 22; 71 x 71 x 36 candidates, tile 20 x 20 x 5 (17.4): 8: 21, 110;
+// 48: 70, 120; 96: 132, 133; 128: 172, 142.
+#define HARD_TILED 5
 __global__ void __launch_bounds__(256)
 k_hard_maps(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
   const IqQuery q = qs[blockIdx.y];
   const IqStep& st = D->steps[q.step];
-  if (!q.multi || q.rep != q.slot || !st.hard) return;
+  if (!q.multi || q.rep != q.slot || !st.hard || st.hcnt >= D->hard_min) return;
   const IqGeo& g = D->g;
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= g.P) return;
@@ -1438,7 +1443,7 @@ k_hard_maps_tiled(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
   extern __shared__ double mreg[];
   const IqQuery q = qs[blockIdx.y];
   const IqStep& st = D->steps[q.step];
-  if (!q.multi || q.rep != q.slot || !st.hard) return;
+  if (!q.multi || q.rep != q.slot || !st.hard || st.hcnt < D->hard_min) return;
   const IqGeo& g = D->g;
   const int nbx = (g.dist[0] + MT_X - 1) / MT_X, nby = (g.dist[1] + MT_Y - 1) / MT_Y;
   const int bx = blockIdx.x % nbx, by = (blockIdx.x / nbx) % nby, cz = blockIdx.x / (nbx * nby);
