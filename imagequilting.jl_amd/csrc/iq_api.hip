@@ -1578,7 +1578,7 @@ void run_batch(iq_plan* pl, const IqQuery* hq, const IqQuery* q, int nq, bool ha
         hipLaunchKernelGGL((k_hard_maps_tiled<16, 16>), dim3(nb, nq), dim3(256), pl->hard_lds, s, D, q);
       HCL();
     }
-    hipLaunchKernelGGL(k_relax_finalize, dim3(nq), dim3(FB), 0, s, D, q);
+    hipLaunchKernelGGL(P >= KS_MIN ? k_relax_finalize<true> : k_relax_finalize<false>, dim3(nq), dim3(FB), 0, s, D, q);
     HCL();
   }
   if (pl->prof) {
@@ -3019,7 +3019,7 @@ int iq_relaxation(iq_ctx* ctx, const double* D, const double* const* Ds, int nau
     HC(hipMemsetAsync(err, 0, sizeof(int32_t), s));
     uint64_t* lkey = m.alloc<uint64_t>(n);
     int32_t* lidx = m.alloc<int32_t>(n);
-    hipLaunchKernelGGL(k_relax_host, dim3(1), dim3(FB), 0, s, n, nsrc, dmaps, tol, bits, ev, lkey, lidx, cnt, err);
+    hipLaunchKernelGGL(n >= KS_MIN ? k_relax_host<true> : k_relax_host<false>, dim3(1), dim3(FB), 0, s, n, nsrc, dmaps, tol, bits, ev, lkey, lidx, cnt, err);
     HCL();
     int32_t code = 0;
     int64_t c = 0;

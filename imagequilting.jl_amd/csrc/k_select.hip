@@ -625,9 +625,9 @@ k_band_finalize(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, int
 #define KS_CAP 512          // bins this small are ranked pairwise in LDS
 #define KS_SAMPLE 4096      // sample of a map from which its order statistic is bracketed
 // Smaller maps are selected without a sample.  A realization with one soft
-// variable, ms without and with the sample by candidates: 40,000: 7.7, 8.9;
-// 44,944: 8.2, 9.2; 49,729: 8.6, 9.2; 55,696: 8.9, 8.9; 59,536: 9.4, 8.9; 71,824:
-// 10.3, 9.4; 147,456: 16.6, 13.5; 262,144: 26.0, 19.5.
+// variable, ms without and with the sample by candidates: 40,000: 7.5, 8.9;
+// 49,729: 8.4, 9.2; 59,536: 9.2, 9.0; 65,536: 9.4, 8.9; 71,824: 10.1, 9.4; 99,856:
+// 12.5, 10.9 (an image of codes: 59,536: 9.2, 9.4; 65,536: 9.6, 9.6; 99,856: 12.8, 11.7).
 #define KS_MIN 57344
 #define KS_U 8              // loads in flight per work-item in the passes over a map
 #define KS_LDS_WORDS 3072   // 64-bit LDS words: histogram 2048 x u32, then the sample (u32), or KS_CAP values and indices
@@ -833,7 +833,6 @@ __device__ __forceinline__ void blk_prefix_bits(const double* __restrict__ map, 
 __device__ __forceinline__ bool blk_prefix_sampled(const double* __restrict__ map, int64_t P, int64_t m, uint32_t* __restrict__ bits,
                                                    uint64_t* __restrict__ lkey, int32_t* __restrict__ lidx, uint64_t* lds,
                                                    SelScratch& sh) {
-  if (P < KS_MIN) return false;
   uint32_t* hist = (uint32_t*)lds;
   uint32_t* smp = (uint32_t*)(lds + 1024);
   const auto* mg = iq_glob(map);
@@ -994,15 +993,21 @@ __device__ __forceinline__ bool blk_prefix_sampled(const double* __restrict__ ma
   return true;
 }
 
-// One word of a prefix set's bits (past the vector cache: set by atomics).
+// One word of a prefix set's bits (SAMPLED: past the vector cache, for it may
+// have been set by atomics).
+template <bool SAMPLED>
 __device__ inline uint32_t ks_word(const uint32_t* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if constexpr (SAMPLED) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else return *p;
 }
 
 // The prefix set of length m as bits.
+template <bool SAMPLED>
 __device__ __forceinline__ void blk_prefix(const double* __restrict__ map, int64_t P, int64_t m, uint32_t* __restrict__ bits,
                                            uint64_t* lkey, int32_t* lidx, uint64_t* lds, SelScratch& sh) {
-  if (m > 0 && blk_prefix_sampled(map, P, m, bits, lkey, lidx, lds, sh)) return;
+  if constexpr (SAMPLED) {
+    if (m > 0 && blk_prefix_sampled(map, P, m, bits, lkey, lidx, lds, sh)) return;
+  }
   uint64_t tv = 0;
   int64_t ti = -1;  // empty prefix
   if (m > 0) blk_kth_key(map, P, m, lds, sh, &tv, &ti);
@@ -1012,6 +1017,10 @@ __device__ __forceinline__ void blk_prefix(const double* __restrict__ map, int64
 
 // Returns the size of the database written to ev (ascending), -1 if every
 // candidate is disabled.  lds: KS_LDS_WORDS 64-bit words; lkey, lidx: P each.
+// SAMPLED: for P >= KS_MIN.  The kernels are built without it as well: with the
+// sampled selection they need more registers than there are, which cost small
+// maps a seventh of their time (1,073 values: 64 us a launch without, 74 with).
+template <bool SAMPLED>
 __device__ __forceinline__ int64_t relax_db(int64_t P, int nsrc, const double* const* maps, double tol, uint32_t* bits, int32_t* ev,
                             uint64_t* lkey, int32_t* lidx, uint64_t* lds, SelScratch& sh) {
   __shared__ int64_t lenj[IQ_MAX_AUX + 2];
@@ -1047,14 +1056,14 @@ __device__ __forceinline__ int64_t relax_db(int64_t P, int nsrc, const double* c
       // the prefix only grows (frac does); an unchanged length keeps its bitmap
       const int64_t len = j == 0 ? dbsize : softdbsize;
       if (len != lenj[j]) {
-        blk_prefix(maps[j], P, len < P ? len : P, bits + j * nwd, lkey, lidx, lds, sh);
+        blk_prefix<SAMPLED>(maps[j], P, len < P ? len : P, bits + j * nwd, lkey, lidx, lds, sh);
         if (threadIdx.x == 0) lenj[j] = len;
       }
       if (j == 0) continue;
       int64_t lc = 0;
       for (int64_t w = threadIdx.x; w < nwd; w += FB) {
-        uint32_t x = ks_word(bits + w);
-        for (int k = 1; k <= j; k++) x &= ks_word(bits + k * nwd + w);
+        uint32_t x = ks_word<SAMPLED>(bits + w);
+        for (int k = 1; k <= j; k++) x &= ks_word<SAMPLED>(bits + k * nwd + w);
         lc += __builtin_popcount(x);
       }
       cnt = blk_sum_i64(lc, sh);
@@ -1068,15 +1077,15 @@ __device__ __forceinline__ int64_t relax_db(int64_t P, int nsrc, const double* c
   const int64_t w0 = threadIdx.x * per, w1 = (w0 + per < nwd) ? w0 + per : nwd;
   int64_t lc = 0;
   for (int64_t w = w0; w < w1; w++) {
-    uint32_t x = ks_word(bits + w);
-    for (int k = 1; k < nsrc; k++) x &= ks_word(bits + k * nwd + w);
+    uint32_t x = ks_word<SAMPLED>(bits + w);
+    for (int k = 1; k < nsrc; k++) x &= ks_word<SAMPLED>(bits + k * nwd + w);
     lc += __builtin_popcount(x);
   }
   int64_t nev;
   int64_t off = blk_excl_scan(lc, &nev, sh);
   for (int64_t w = w0; w < w1; w++) {
-    uint32_t x = ks_word(bits + w);
-    for (int k = 1; k < nsrc; k++) x &= ks_word(bits + k * nwd + w);
+    uint32_t x = ks_word<SAMPLED>(bits + w);
+    for (int k = 1; k < nsrc; k++) x &= ks_word<SAMPLED>(bits + k * nwd + w);
     while (x) {
       int b = __builtin_ctz(x);
       x &= x - 1;
@@ -1089,7 +1098,8 @@ __device__ __forceinline__ int64_t relax_db(int64_t P, int nsrc, const double* c
 
 // Multi-source finalize: relaxation + tau model + draw (iqsim.jl:230-243).
 // Source order: hard tile -> [hard, overlap, soft...], else [overlap, soft...].
-extern "C" __global__ void __launch_bounds__(FB)
+template <bool SAMPLED>
+__global__ void __launch_bounds__(FB)
 k_relax_finalize(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
   __shared__ SelScratch sh;
   __shared__ double sv[IQ_SORT_MAX];
@@ -1118,7 +1128,7 @@ k_relax_finalize(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs) {
   __syncthreads();
   int32_t* ev = D->ev + slot * g.P;
   // list scratch: the slot's key and superset lists (used later, by the ranks of a large database)
-  const int64_t nev = relax_db(g.P, nsrc, mp, D->tol, D->bits + slot * D->nmap * D->nw32, ev,
+  const int64_t nev = relax_db<SAMPLED>(g.P, nsrc, mp, D->tol, D->bits + slot * D->nmap * D->nw32, ev,
                                (uint64_t*)(D->rkey + slot * 2 * g.P), D->sup + slot * g.P, (uint64_t*)sv, sh);
   if (nev < 0) {
     if (threadIdx.x == 0) { set_err(D->err, IQ_KERR_NOCAND); *o.pick = -2; }
@@ -1162,13 +1172,14 @@ k_band_pick_host(const double* __restrict__ Dm, int64_t n, double tol, int32_t* 
   if (threadIdx.x == 0) *count = tot;
 }
 
-extern "C" __global__ void __launch_bounds__(FB)
+template <bool SAMPLED>
+__global__ void __launch_bounds__(FB)
 k_relax_host(int64_t P, int nsrc, const double* const* __restrict__ maps, double tol, uint32_t* __restrict__ bits,
              int32_t* __restrict__ ev, uint64_t* __restrict__ lkey, int32_t* __restrict__ lidx, int64_t* __restrict__ count,
              int32_t* __restrict__ err) {
   __shared__ SelScratch sh;
   __shared__ uint64_t ks[KS_LDS_WORDS];
-  const int64_t n = relax_db(P, nsrc, maps, tol, bits, ev, lkey, lidx, ks, sh);
+  const int64_t n = relax_db<SAMPLED>(P, nsrc, maps, tol, bits, ev, lkey, lidx, ks, sh);
   if (threadIdx.x == 0) {
     if (n < 0) set_err(err, IQ_KERR_NOCAND);
     *count = n < 0 ? 0 : n;
