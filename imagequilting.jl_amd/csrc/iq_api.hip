@@ -466,6 +466,7 @@ struct iq_plan {
   int hard_bx = 16;        // candidate block width of the tiled maps (32 or 16; 16 rows)
   size_t maps_lds = 0;     // LDS of the exact maps (k_maps_mfma), 0: not used by the plan
   int maps_steps = 0;      // most steps of any voxel list
+  double maps_gather = 0;  // window voxels (queries x candidates x voxels) of a batch below which its maps are gathered
   IqMapTile* dm = nullptr;   // map tiles (all batches of a run)
   int64_t dm_cap = 0;
   double* mpack = nullptr;   // their query values in fragment order (one batch at a time)
@@ -654,6 +655,15 @@ void tune_scan(iq_plan* pl) {
   if ((int)hq.size() <= 32) pl->nw_tiles[2] = pl->nw_tiles[1];
   for (hipEvent_t e : ev) HC(hipEventDestroy(e));
 }
+
+// A batch's exact maps are gathered below this much work (window voxels:
+// candidates times voxels, summed over the maps).  The matrix cores want steps
+// enough for their groups and queries enough for their tiles of four: with one
+// soft variable, ms a realization gathered and on the matrix cores, by window
+// voxels of a wave: 0.4M (48x40 image, tile 12x12): 1.77, 1.88; 4M (100x100,
+// 16x16): 1.94, 2.09; 7M (128x128, 16x16): 2.28, 2.41; 40M (200x200, 24x24): 4.29,
+// 4.27; from 64M on they are up to 7 % slower gathered, then more.
+#define MAPS_GATHER 32e6
 
 // Voxel lists of the exact maps (k_maps.hip): every mask's, then the whole
 // tile's, cut into chunks whose window region fits MM_LDS (whole planes, as
@@ -1286,6 +1296,12 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
   H.nmap = nmap;
   H.nw32 = nw32;
   if (pl->any_multi || (!pl->fast && !hmasks.empty())) build_map_lists(pl, tvox, full_off, s);
+  // IQHIP_MAPS=gather or matrix: all exact maps that way
+  pl->maps_gather = MAPS_GATHER;
+  if (const char* em = std::getenv("IQHIP_MAPS")) {
+    if (std::string(em) == "gather") pl->maps_gather = HUGE_VAL;
+    if (std::string(em) == "matrix") pl->maps_gather = 0.0;
+  }
   if (pl->any_multi) {
     // hard-data maps: the tiles from hard_min points on are made by the tiled
     // kernel where the candidate block's training-image region fits in LDS
@@ -1420,7 +1436,7 @@ enum { SEL_SCAN = 0, SEL_LEARNED = 1, SEL_CHECK = 2 };
 
 template <typename T>
 void run_batch(iq_plan* pl, const IqQuery* hq, const IqQuery* q, int nq, bool has_plain, bool has_multi, int sel,
-               const int4* tiles, const int4* htiles, int ntiles, const IqMapTile* mtiles, int nmtiles) {
+               const int4* tiles, const int4* htiles, int ntiles, const IqMapTile* mtiles, int nmtiles, int mq) {
   const IqGeo& g = pl->geo;
   hipStream_t s = pl->ctx->stream;
   const IqDev* D = pl->dd;
@@ -1435,7 +1451,11 @@ void run_batch(iq_plan* pl, const IqQuery* hq, const IqQuery* q, int nq, bool ha
     hipLaunchKernelGGL((k_query_prep<T>), dim3(nq, nsrc_prep), dim3(256), 0, s, D, q);
   }
   HCL();
-  if (nmtiles > 0) {
+  if (nmtiles > 0 && mq > 0) {
+    // few exact maps (map_tiles): gathered
+    hipLaunchKernelGGL(k_maps_gather, dim3(nblk(P, 64), nmtiles, mq), dim3(64), 0, s, D, q, mtiles);
+    HCL();
+  } else if (nmtiles > 0) {
     // exact maps on the matrix cores: the overlap and soft sources of the
     // multi-source queries, the overlap of plain queries the scans do not take
     hipLaunchKernelGGL(k_maps_pack, dim3(pl->maps_steps, nmtiles), dim3(256), 0, s, D, q, mtiles, pl->mpack, pl->maps_steps);
@@ -1614,6 +1634,7 @@ struct RunBatch {
   int nt;
   int64_t moff;  // map tiles [moff, moff + nm)
   int nm;
+  int mq;        // most queries of a tile where the maps are gathered, 0: on the matrix cores
 };
 template <typename T>
 void plan_run_launches(iq_plan* pl, const std::vector<IqQuery>& qs, const std::vector<RunBatch>& batches,
@@ -1652,10 +1673,20 @@ void map_tiles(iq_plan* pl, IqQuery* q, RunBatch& bt, std::vector<IqMapTile>& mt
       mtiles.push_back(T);
     }
   };
+  const size_t t0 = mtiles.size();
   for (int a = 0; a < pl->naux; a++) add(2 + a, nm, reps);
   for (int m = nm; m >= 0; m--) add(0, m - 1, multi[m]);
   for (int m = nm; m >= 1; m--) add(-1, m - 1, plain[m]);
   bt.nm = (int)((int64_t)mtiles.size() - bt.moff);
+  bt.mq = 0;
+  double work = 0.0;
+  int most = 0;
+  for (size_t i = t0; i < mtiles.size(); i++) {
+    const IqMapTile& T = mtiles[i];
+    most = std::max(most, (int)T.n);
+    if (T.list >= 0) work += (double)T.n * (double)pl->geo.P * (T.list < nm ? pl->masks[T.list].V : pl->geo.tilevox);
+  }
+  if (work < pl->maps_gather) bt.mq = most;
 }
 
 // The query table of a run: wave k of every grid, all realizations, in
@@ -1691,7 +1722,7 @@ void plan_tables(iq_plan* pl, const double* uniforms, const int64_t* forced, boo
         return pl->steps[a.step].mask < pl->steps[b.step].mask;
       });
     for (size_t b0 = 0; b0 < wq.size(); b0 += (size_t)pl->nslots) {
-      RunBatch bt{(int64_t)qs.size(), 0, false, false, 0, 0, 0, 0};
+      RunBatch bt{(int64_t)qs.size(), 0, false, false, 0, 0, 0, 0, 0};
       const size_t b1 = std::min(wq.size(), b0 + (size_t)pl->nslots);
       std::vector<size_t> order(b1 - b0);
       for (size_t k = b0; k < b1; k++) order[k - b0] = k;
@@ -1749,7 +1780,8 @@ void upload_map_tiles(iq_plan* pl, const std::vector<IqMapTile>& mtiles, const s
     pl->dm_cap = (int64_t)mtiles.size();
   }
   int64_t widest = 0;
-  for (const RunBatch& b : batches) widest = std::max<int64_t>(widest, b.nm);
+  for (const RunBatch& b : batches)
+    if (b.mq == 0) widest = std::max<int64_t>(widest, b.nm);
   if (widest > pl->mpack_cap) {
     pl->mpack = pl->mem.alloc<double>((size_t)widest * pl->maps_steps * MM_STEP * MM_Q);
     pl->mpack_cap = widest;
@@ -1882,7 +1914,7 @@ void plan_run_launches(iq_plan* pl, const std::vector<IqQuery>& qs, const std::v
     int sel = SEL_SCAN;
     if (learned && b.plain) sel = (pl->lrn_check > 0 && nplain++ % pl->lrn_check == 0) ? SEL_CHECK : SEL_LEARNED;
     run_batch<T>(pl, qs.data() + b.off, pl->dq + b.off, b.n, b.plain, b.multi, sel, pl->dt + b.toff,
-                 tiles.data() + b.toff, b.nt, pl->dm + b.moff, b.nm);
+                 tiles.data() + b.toff, b.nt, pl->dm + b.moff, b.nm, b.mq);
     if (sel == SEL_CHECK) {
       // the full scan decided this batch: stop using the shortlist once its
       // cumulative recall on the exact bands falls below the threshold.  The
@@ -2502,7 +2534,7 @@ void conv_harvest(iq_plan* pl, int64_t nq_total, int topn, int nhard, int nrand,
       if (!pool.empty()) harvest_queries<T>(pl, pool, topn, nrand, rng, ws, set);
     }
     run_batch<T>(pl, qs.data() + bt.off, pl->dq + bt.off, bt.n, bt.plain, bt.multi, SEL_SCAN, nullptr, nullptr, 0, pl->dm + bt.moff,
-                 bt.nm);
+                 bt.nm, bt.mq);
   }
   HC(hipStreamSynchronize(s));
   int32_t code = 0;

@@ -199,6 +199,76 @@ k_maps_mfma(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, const I
   }
 }
 
+// The chain of one candidate over V listed voxels: offsets and query values
+// come through LDS, MG_DEEP window values are in flight at once.  `img` is the
+// image at the candidate's first voxel.
+#define MG_DEEP 64
+#define MG_CHUNK 1024
+template <typename T>
+__device__ __forceinline__ double gather_chain(const T* img_, const int32_t* toff, const double* kv, int V, int32_t* ol, double* kl) {
+  const auto img = iq_glob(img_);
+  double ab = 0.0;
+  for (int j0 = 0; j0 < V; j0 += MG_CHUNK) {
+    const int n = V - j0 < MG_CHUNK ? V - j0 : MG_CHUNK;
+    if (j0) __syncthreads();  // the previous chunk is no longer read
+    for (int k = threadIdx.x; k < (n + MG_DEEP - 1) / MG_DEEP * MG_DEEP; k += (int)blockDim.x) {
+      ol[k] = k < n ? toff[j0 + k] : 0;
+      kl[k] = k < n ? kv[j0 + k] : 0.0;
+    }
+    __syncthreads();
+    for (int k0 = 0; k0 < n; k0 += MG_DEEP) {
+      T t[MG_DEEP];
+#pragma unroll
+      for (int i = 0; i < MG_DEEP; i++) t[i] = img[ol[k0 + i]];
+      if (k0 + MG_DEEP <= n) {
+#pragma unroll
+        for (int i = 0; i < MG_DEEP; i++) ab = __builtin_fma((double)t[i], kl[k0 + i], ab);
+      } else {  // past the list: zero times zero, whatever the image holds
+#pragma unroll
+        for (int i = 0; i < MG_DEEP; i++) ab = __builtin_fma(k0 + i < n ? (double)t[i] : 0.0, kl[k0 + i], ab);
+      }
+    }
+  }
+  return ab;
+}
+
+// The same maps, of little work: a work-item per candidate gathers its window
+// from the image, a query at a time, in one launch.  What bounds it is the
+// latency of the loads of the few wavefronts there are, so groups are of one,
+// over as many compute units as they reach (4,232 candidates, 192 voxels: 13.8
+// us in groups of four, 10.2 of one; k_maps_pack and k_maps_mfma 15.6).  Grid:
+// (candidate blocks, tiles, queries of a tile).
+__global__ void __launch_bounds__(64)
+k_maps_gather(const IqDev* __restrict__ D, const IqQuery* __restrict__ qs, const IqMapTile* __restrict__ tiles) {
+  __shared__ int32_t ol[MG_CHUNK];
+  __shared__ double kl[MG_CHUNK];
+  const IqMapTile& T = tiles[blockIdx.y];
+  if ((int)blockIdx.z >= T.n) return;
+  const IqGeo& g = D->g;
+  const int64_t slot = qs[T.q[blockIdx.z]].slot;
+  const int src = T.src < 0 ? 0 : T.src;
+  const int64_t c0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t c = c0 < g.P ? c0 : g.P - 1;
+  const int cx = (int)(c % g.dist[0]), cy = (int)((c / g.dist[0]) % g.dist[1]);
+  const int cz = (int)(c / ((int64_t)g.dist[0] * g.dist[1]));
+  const int64_t at = iq_lin3(g.ti, cx, cy, cz);
+  const double* kv = D->kv + slot * D->kv_stride + (int64_t)src * g.tilevox;
+  double a2 = 0.0, ab = 0.0;
+  if (T.src >= 2) {
+    a2 = D->a2soft[T.src - 2][c];
+    ab = gather_chain(D->auxti[T.src - 2] + at, D->toff + D->full_off, kv, g.tilevox, ol, kl);
+  } else if (T.list >= 0) {
+    const IqMask& m = D->masks[T.list];
+    a2 = D->a2maps[m.a2][c];
+    if (D->ti_f32) ab = gather_chain((const float*)D->ti + at, D->toff + m.off, kv, m.V, ol, kl);
+    else ab = gather_chain((const double*)D->ti + at, D->toff + m.off, kv, m.V, ol, kl);
+  }
+  if (c0 >= g.P) return;
+  const double b2 = D->b2[slot * (2 + D->naux) + src];
+  double* out = T.src < 0 ? D->dexact + slot * g.P : D->maps + (slot * D->nmap + src) * g.P;
+  out[c] = D->disabled[c] ? __builtin_inf() : __builtin_fabs((a2 - 2.0 * ab) + b2);
+}
+
 // Plain queries whose training image the FP32 scans do not take (values out
 // of range, or Float64 values dominated by a common offset): their overlap
 // maps are exact for every candidate (k_maps_mfma), all enabled candidates
