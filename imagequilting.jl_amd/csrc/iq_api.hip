@@ -337,7 +337,9 @@ bool fits_f32(const double* v, int64_t n) {
 // by it is exact, and the interval keeps its share of the distances.  (64x64x32
 // image times 1e-18, tile 14x14x5: every window rechecked and 162 ms a
 // realization without it, 8 windows and 10 ms with it.)
-bool scan_takes_rounded(const double* v, int64_t n, double* scale) {
+// Where windows are disabled the image holds zeros that no distance sees
+// (inactive voxels): only the first and last voxels of the others count.
+bool scan_takes_rounded(const double* v, int64_t n, const IqGeo& g, const uint8_t* disabled, double* scale) {
   double mx = 0.0;
   for (int64_t i = 0; i < n; i++) {
     const double x = v[i];
@@ -345,13 +347,25 @@ bool scan_takes_rounded(const double* v, int64_t n, double* scale) {
     mx = std::max(mx, std::fabs(x));
   }
   *scale = mx > 0.0 && mx < 1.0 ? std::ldexp(1.0, -std::ilogb(mx)) : 1.0;
-  double s1 = 0.0, s2 = 0.0;
-  for (int64_t i = 0; i < n; i++) {
-    const double x = v[i] * *scale;
+  double s1 = 0.0, s2 = 0.0, cnt = 0.0;
+  auto add = [&](double x) {
+    x *= *scale;
     s1 += x;
     s2 += x * x;
+    cnt += 1.0;
+  };
+  if (std::find_if(disabled, disabled + g.P, [](uint8_t d) { return d != 0; }) == disabled + g.P) {
+    for (int64_t i = 0; i < n; i++) add(v[i]);
+  } else {
+    const int64_t last = iq_lin3(g.ti, g.tile[0] - 1, g.tile[1] - 1, g.tile[2] - 1);
+    for (int64_t c = 0; c < g.P; c++) {
+      if (disabled[c]) continue;
+      const int64_t at = iq_lin3(g.ti, c % g.dist[0], c / g.dist[0] % g.dist[1], c / ((int64_t)g.dist[0] * g.dist[1]));
+      add(v[at]);
+      add(v[at + last]);
+    }
   }
-  const double m = s1 / (double)n, q = s2 / (double)n;
+  const double m = s1 / cnt, q = s2 / cnt;
   return q <= 32.0 * (q - m * m);
 }
 bool fits_range(const float* v, int64_t n) {
@@ -994,7 +1008,7 @@ void plan_build(iq_ctx* ctx, const iq_plan_desc* descs, int ngrid, iq_plan* pl) 
   } else {
     H.ti = pl->mem.upload(tid, tivox, s);
     pl->fast = fits_f32(tid, tivox);
-    if (!pl->fast) pl->fast = pl->rounded = scan_takes_rounded(tid, tivox, &H.scan_s);
+    if (!pl->fast) pl->fast = pl->rounded = scan_takes_rounded(tid, tivox, g, d->disabled, &H.scan_s);
     if (!pl->rounded) H.scan_s = 1.0;
     H.scan_s2 = H.scan_s * H.scan_s;
     if (pl->fast) {

@@ -37,3 +37,20 @@ def test_wide_superset_matches_oracle(nreal):
     T = np.random.default_rng(73).standard_normal((60, 57))
     print("white noise, realizations", nreal, flush=True)
     _compare(T, (8, 8), (20, 22), overlap=(0.25, 0.25), tol=1.0, nreal=nreal)
+
+
+@pytest.mark.parametrize("offset,scanned", [(2000.0, False), (0.0, True), (0.2, True)], ids=["depth", "centred", "porosity"])
+def test_inactive_voxels_do_not_hide_an_offset(offset, scanned):
+    """The zeros in place of inactive voxels make the variance of a far-off
+    image look large; no window that counts holds one."""
+    T = _smooth(np.random.default_rng(74), (64, 61), 5, np.float64)
+    T = offset + (50.0 if offset > 1 else 0.05) * T / T.std()
+    T[:14, :20] = np.nan
+    kw = dict(overlap=(0.2, 0.25))
+    plan, _ = iqhip.make_plan(T, (13, 12), (70, 64), rng=np.random.default_rng(1), **kw)
+    plan.run(np.random.default_rng(2).random((1, plan.npath)))
+    queries, members, band = plan.select_stats()
+    plan.close()
+    assert queries > 0 and band > 0 and (members > 0) == scanned  # the exhaustive map counts no superset
+    print("offset", offset, flush=True)
+    _compare(T, (13, 12), (70, 64), **kw)
