@@ -823,7 +823,7 @@ __device__ __forceinline__ void blk_prefix_bits(const double* __restrict__ map, 
 // statistic is found in the list, whose members then get their bits.  The
 // passes over the maps are what the relaxation costs, and the radix selection
 // takes four: 336 queries of 3 maps of 216,225 values took 988 us that way,
-// 684 us this way (the bits and the list are what a pass writes).  Ties (maps of
+// 579 us this way (the bits and the list are what a pass writes).  Ties (maps of
 // codes, of few hard points) are known by value from the list, or from one
 // counting pass where the bracket is a single value; the radix selection goes
 // through every digit of them.  Two maps of 216,225 values in 40 and 3 levels:
