@@ -598,8 +598,8 @@ void launch_scan_mfma(iq_plan* pl, const IqQuery* q, int nq, int nw, bool list, 
 
 // Scan autotuner: the MFMA scan's group size (2, 3 or 4 wavefronts) is measured
 // on the plan itself.  A batch of the plan's own masked steps (32 queries,
-// then up to 64 as the slots allow) is prepared once; each group size runs one
-// warm-up and three timed launches (the least counts: a launch timed by itself
+// then up to 64 as the slots allow) is prepared once; after a warm-up each group
+// size runs three timed launches (the least counts: a launch timed by itself
 // may be late); the fastest size is kept per tile count.  What a listing scan
 // writes depends on the bound and the list it starts from, so both are reset
 // before every launch, outside the time taken (an image of ties, 301,806
@@ -644,16 +644,17 @@ void tune_scan(iq_plan* pl) {
     hipLaunchKernelGGL(k_mfma_bprep, dim3(pl->hd.ktab.nstep, ntile), dim3(64), 0, s, D, dq, nq);
     HCL();
     float best = 1e30f;
+    launch_scan_mfma(pl, dq, nq, nwa[0], scan_lists(pl, nq, nwa[0]), s);  // warm-up
     for (int nw : nwa) {
       const bool list = scan_lists(pl, nq, nw);
-      for (int rep = -1; rep < 3; rep++) {
+      for (int rep = 0; rep < 3; rep++) {
         if (list) {  // the queries' slots are 0 to nq - 1
           hipLaunchKernelGGL(k_scan_reset, dim3(1), dim3(64), 0, s, D, nq);
           HCL();
         }
-        if (rep >= 0) HC(hipEventRecord(ev[2 * rep], s));
+        HC(hipEventRecord(ev[2 * rep], s));
         launch_scan_mfma(pl, dq, nq, nw, list, s);
-        if (rep >= 0) HC(hipEventRecord(ev[2 * rep + 1], s));
+        HC(hipEventRecord(ev[2 * rep + 1], s));
       }
       HC(hipEventSynchronize(ev[5]));
       float us = 1e30f;
